@@ -19,11 +19,12 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libkernrt_hip.so")
 
-SOURCES = ["kernels.hip", "gemm.hip", "attn_mx.hip", "backend.hip", "llm.cpp"]
+SOURCES = ["kernels.hip", "gemm.hip", "gemm_direct.hip", "attn_mx.hip", "backend.hip", "llm.cpp"]
 # per-source extra flags: the matrix-core attention and the Q8_0 GEMM keep
 # MFMA results in ordinary vector registers (their vector epilogues read them
 # directly)
-EXTRA = {"attn_mx.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+EXTRA = {"attn_mx.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+         "gemm_direct.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 FLAGS = [
     "-O3", "-std=c++17", "--offload-arch=gfx950", "-fPIC", "-shared",

@@ -105,9 +105,81 @@ __device__ __forceinline__ float scale_value(bool f16, uint32_t bits) {
     return f16 ? f16w((uint16_t)bits) : u2f(bits);
 }
 
+// Workgroup ids are dispatched round-robin over the 8 XCDs; consecutive
+// logical tiles (the row tiles of one column tile) go to one XCD and share
+// its L2.
+__device__ __forceinline__ uint32_t gemm_xcd_tile(uint32_t id, uint32_t count) {
+    const uint32_t per = count >> 3, rem = count & 7, xcd = id & 7, k = id >> 3;
+    return xcd < rem ? xcd * (per + 1) + k : rem * (per + 1) + (xcd - rem) * per + k;
+}
+
+// SWI: the gate/up launch of a SwiGLU FFN with SiLU(gate) * up and its Q8
+// blocks as the epilogue (silu_quant's arithmetic, elementwise.rs / quant.rs:
+// 864-873): the tile's 64 columns are gate rows 32 t .. 32 t + 31 (ms.q[0])
+// and up rows 32 t .. 32 t + 31 (ms.q[1]) of the same hidden block t, and the
+// outputs are h's int8 quants and block scales in `so` instead of f32 gate/up,
+// in chain-major block order when `cm` is set (for a chain-split down).
+struct SwiOut {
+    int8_t* q;
+    float* s;
+    uint16_t* h;
+    uint32_t cm;
+};
+
+// ROPE: the q/k/v launch of a prefill with head_dim 64 (one head per 64-column
+// tile) and the half-split RoPE layout: the epilogue rotates each q and k
+// head's pairs (i, i + 32) at the row's position, as k_rope_kv does
+// (cpu.rs:664-705), writes q to y[0], and k and v straight into the KV cache
+// at the row's slot (kv_write, cpu.rs:563-573); y[1] and y[2] are not written.
+struct RopeOut {
+    const uint32_t* pos;    // [M] positions
+    const uint32_t* slots;  // [M] cache slots
+    const float2* tab;      // (cos, sin) per (position, pair): [pos][32]
+    float* kc;              // the layer's keys: [seq_len][kv_dim]
+    float* vc;              // and values
+    uint32_t kv_dim;
+};
+
+// SWI: hidden column 32 blk + c of row m from its gate and up projections; the
+// 32 lanes of a half-wave hold one row's block and all call this.
+__device__ __forceinline__ void swi_out(const SwiOut& so, float g, float u, uint32_t m, uint32_t M, uint32_t hidden,
+                                        uint32_t blk, uint32_t c, const uint64_t* etab) {
+    // cpu.rs:708-710: silu(g) * u
+    const float h = div_rn(g, 1.0f + glibc_expf(-g, etab)) * u;
+    const uint32_t nbh = hidden >> 5, pb = so.cm ? cm_block(blk, nbh) : blk;
+    const size_t row = m < M ? m : 0, oi = row * hidden + pb * 32 + c, si = row * nbh + pb;
+    quant_lane(h, m < M, so.q + oi, so.s + si, so.h + si);
+}
+
+// ROPE: columns h0 + i and h0 + i + 32 of row m < M of q (mi 0), k or v (2).
+__device__ __forceinline__ void rope_out(const RopeOut& ro, int mi, float* q, uint32_t ldq, float a, float b,
+                                         uint32_t m, uint32_t h0, uint32_t i) {
+    float r0 = a, r1 = b;
+    if (mi != 2) {  // k_rope_kv: r0 = a cos - b sin, r1 = a sin + b cos
+        const float2 cs = ro.tab[(size_t)ro.pos[m] * 32 + i];
+        r0 = a * cs.x - b * cs.y;
+        r1 = a * cs.y + b * cs.x;
+    }
+    float* dst = (mi == 0 ? q + (size_t)m * ldq : (mi == 1 ? ro.kc : ro.vc) + (size_t)ro.slots[m] * ro.kv_dim) + h0 + i;
+    dst[0] = r0;
+    dst[32] = r1;
+}
+
 // The four-partial Q8_0 GEMM (gemm.hip) over a matrix set, rows >= 8.
 hipError_t launch_gemm_q8(hipStream_t st, int sem, const MatSet& ms, size_t k, QuantAct x, size_t rows,
                           int32_t* dbg);
+// The same for either epilogue and any row count, every wave staging its own
+// operands (gemm_direct.hip): few rows or narrow outputs. _swi and _rope: the
+// gate/up and q/k/v launches with their epilogues.
+hipError_t launch_gemm_direct(hipStream_t st, int sem, const MatSet& ms, size_t k, QuantAct x, size_t rows,
+                              int32_t* dbg);
+hipError_t launch_direct_swi(hipStream_t st, int sem, const MatSet& ms, size_t k, QuantAct x, size_t rows, SwiOut so);
+hipError_t launch_direct_rope(hipStream_t st, int sem, const MatSet& ms, size_t k, QuantAct x, size_t rows,
+                              RopeOut ro);
+// The Q8_0x4 forms by grid: direct up to kDirectTiles16 16x16 units (one wave
+// each), then 64x64 tiles (a 32x32 unit per wave) up to kChainTiles64 of them,
+// then 128x128 tiles (32x64 per wave).
+static constexpr size_t kDirectTiles16 = 1408, kChainTiles64 = 640, kDirectSwiMax = 256, kDirectRopeMax = 400;
 
 // The chunk pipeline shared by both GEMM kernels. At chunk c, the register
 // stage (c + 1) % NS holds chunk c + 1 and LDS buffer c & 1 holds chunk c.

@@ -1,5 +1,5 @@
-// Q8_0 GEMM with the reference's four partial sums (dot.rs:34-45), for
-// prefill and batched rows (M >= 8). Built as its own translation unit with
+// Q8 GEMM for prefill and batched rows: Q8_0 with the reference's four partial
+// sums (dot.rs:34-45) and Q8_0x4 with its FMA chain (quant.rs:276-288). Built as its own translation unit with
 // -mllvm -amdgpu-mfma-vgpr-form=1, so that MFMA results land in ordinary
 // vector registers, where the epilogue reads them.
 //
@@ -27,6 +27,9 @@
 // outer product puts the scale product of the same output in the same
 // register of its half.
 //
+// A Q8_0x4 output is one chain, slot = fma(isum, sa * sb, slot), so a wave sums
+// its sub-tile over every block (SEM_FMA_CHAIN, CPW 4, one accumulator set).
+//
 // Operands are staged through LDS in chunks of KC blocks: every row's KC*32
 // bytes by coalesced 16-byte loads, NS chunks ahead in registers, into a
 // double-buffered tile whose rows are padded by 16 bytes (the fragment reads
@@ -46,41 +49,6 @@ namespace kr {
 typedef int g_v4i __attribute__((ext_vector_type(4)));
 typedef int g_v16i __attribute__((ext_vector_type(16)));
 typedef float g_v32f __attribute__((ext_vector_type(32)));
-
-// Workgroup ids are dispatched round-robin over the 8 XCDs; consecutive
-// logical tiles (the row tiles of one column tile) go to one XCD and share
-// its L2.
-__device__ __forceinline__ uint32_t gemm_xcd_tile(uint32_t id, uint32_t count) {
-    const uint32_t per = count >> 3, rem = count & 7, xcd = id & 7, k = id >> 3;
-    return xcd < rem ? xcd * (per + 1) + k : rem * (per + 1) + (xcd - rem) * per + k;
-}
-
-// SWI: the gate/up launch of a SwiGLU FFN with SiLU(gate) * up and its Q8
-// blocks as the epilogue (silu_quant's arithmetic, elementwise.rs / quant.rs:
-// 864-873): the tile's 64 columns are gate rows 32 t .. 32 t + 31 (ms.q[0])
-// and up rows 32 t .. 32 t + 31 (ms.q[1]) of the same hidden block t, and the
-// outputs are h's int8 quants and block scales in `so` instead of f32 gate/up,
-// in chain-major block order when `cm` is set (for a chain-split down).
-struct SwiOut {
-    int8_t* q;
-    float* s;
-    uint16_t* h;
-    uint32_t cm;
-};
-
-// ROPE: the q/k/v launch of a prefill with head_dim 64 (one head per 64-column
-// tile) and the half-split RoPE layout: the epilogue rotates each q and k
-// head's pairs (i, i + 32) at the row's position, as k_rope_kv does
-// (cpu.rs:664-705), writes q to y[0], and k and v straight into the KV cache
-// at the row's slot (kv_write, cpu.rs:563-573); y[1] and y[2] are not written.
-struct RopeOut {
-    const uint32_t* pos;    // [M] positions
-    const uint32_t* slots;  // [M] cache slots
-    const float2* tab;      // (cos, sin) per (position, pair): [pos][32]
-    float* kc;              // the layer's keys: [seq_len][kv_dim]
-    float* vc;              // and values
-    uint32_t kv_dim;
-};
 
 // CS: the chain-split form for launches with few output tiles. Operands
 // are chain-major (each row holds the blocks of chain 0 -- blocks 0, 4, 8,
@@ -107,10 +75,13 @@ __global__ __launch_bounds__(64 * (TM / 32) * (TN / (32 * NJ)) * (4 / CPW), WPE)
     static_assert(NJ == 1 || NJ == 2, "unit columns per wave");
     static_assert(CPW == 1 || CPW == 2 || CPW == 4, "chains per wave");
     static_assert(NT % PPR == 0, "a thread's pieces share their column");
-    static_assert(!SWI || (TN == 64 && NJ == 2 && CPW < 4), "the SwiGLU epilogue needs one gate and one up unit per wave");
-    static_assert(!CS || (CPW == 4 && !SWI && !DBG), "a chain-split wave runs its tile's one chain");
-    static_assert(!ROPE || (TN == 64 && NJ == 2 && CPW < 4 && !SWI && !CS), "a RoPE tile is one 64-wide head");
-    constexpr bool WF16 = SEM == SEM_FOUR_PARTIALS_F16;
+    // ONE: the wave sums all its blocks into one accumulator, in block order
+    constexpr bool FMA = SEM == SEM_FMA_CHAIN, ONE = CS || FMA;
+    static_assert(!SWI || (FMA ? TN % 64 == 0 : TN == 64 && NJ == 2 && CPW < 4), "a hidden block is 32 gate and 32 up columns");
+    static_assert(!CS || (CPW == 4 && !SWI && !DBG && !FMA), "a chain-split wave runs its tile's one chain");
+    static_assert(!FMA || CPW == 4, "the FMA chain is serial over K");
+    static_assert(!ROPE || ((FMA ? TN % 64 == 0 : TN == 64 && NJ == 2 && CPW < 4) && !SWI && !CS), "a RoPE tile is 64-wide heads");
+    constexpr bool WF16 = SEM != SEM_FOUR_PARTIALS_F32;
     __shared__ __align__(16) int8_t lds[LDS_BYTES];
     uint64_t* const etab = (uint64_t*)(lds + RING_BYTES);
     auto sA = [&](int buf) { return lds + buf * BUF_BYTES; };
@@ -126,7 +97,7 @@ __global__ __launch_bounds__(64 * (TM / 32) * (TN / (32 * NJ)) * (4 / CPW), WPE)
     const uint32_t nbr = K >> 5, nb = CS ? nbr / 4 : nbr, nchunks = (nb + KC - 1) / KC;
     const uint32_t kend = nb * 32, koff = chain * kend, soff = chain * nb;
     const int mi_ = SWI ? 0 : nt < ms.tile_end[0] ? 0 : (nt < ms.tile_end[1] ? 1 : 2);
-    const uint32_t m0 = mt * TM, n0 = SWI ? nt * 32 : (nt - (mi_ == 0 ? 0 : ms.tile_end[mi_ > 0 ? mi_ - 1 : 0])) * TN;
+    const uint32_t m0 = mt * TM, n0 = SWI ? nt * (TN / 2) : (nt - (mi_ == 0 ? 0 : ms.tile_end[mi_ > 0 ? mi_ - 1 : 0])) * TN;
     const int8_t* __restrict__ W = ms.q[mi_];
     const void* __restrict__ WS = ms.s[mi_];
     const uint32_t N = ms.n[mi_];
@@ -141,14 +112,15 @@ __global__ __launch_bounds__(64 * (TM / 32) * (TN / (32 * NJ)) * (4 / CPW), WPE)
     // chunk; scale s = tid + NT i is an activation scale (row s / KC, block
     // s % KC) for s < KC TM, else a weight scale. Rows past M or N read the
     // last row, blocks past the row end its last block.
+    auto swi_row = [&](uint32_t c) { return n0 + 32 * (c >> 6) + (c & 31); };
     const int8_t* gp[NP];
     uint32_t lp[NP];
 #pragma unroll
     for (int i = 0; i < NP; i++) {
         const uint32_t q = min(tid + NT * i, (uint32_t)NQ - 1), isb = q >= PPR * TM;
         const uint32_t row = (isb ? q - PPR * TM : q) / PPR;
-        if (SWI)  // B rows 0..31: gate, 32..63: up, of the hidden block's rows
-            gp[i] = isb ? (row >= 32 ? ms.q[1] : ms.q[0]) + (size_t)min(n0 + (row & 31), N - 1) * K
+        if (SWI)  // B rows 64 i + 0..31: gate, + 32..63: up, of hidden block n0 / 32 + i
+            gp[i] = isb ? (row & 32 ? ms.q[1] : ms.q[0]) + (size_t)min(swi_row(row), N - 1) * K
                         : x.q + (size_t)min(m0 + row, M - 1) * K;
         else
             gp[i] = (isb ? W + (size_t)min(n0 + row, N - 1) * K : x.q + (size_t)min(m0 + row, M - 1) * K) + koff;
@@ -170,12 +142,12 @@ __global__ __launch_bounds__(64 * (TM / 32) * (TN / (32 * NJ)) * (4 / CPW), WPE)
             const uint32_t sidx = tid + NT * i;
             const uint32_t blk = soff + min(c * KC + sidx % KC, nb - 1);
             if (sidx < KC * TM) {
-                st.sc[i] = f2u(x.s[(size_t)min(m0 + sidx / KC, M - 1) * nbr + blk]);
+                st.sc[i] = scale_bits(FMA, FMA ? (const void*)x.h : (const void*)x.s, (size_t)min(m0 + sidx / KC, M - 1) * nbr + blk);
             } else if (sidx < KC * (TM + TN)) {
                 const uint32_t col2 = (sidx - KC * TM) / KC;
                 if (SWI)
-                    st.sc[i] = scale_bits(WF16, col2 >= 32 ? ms.s[1] : ms.s[0],
-                                          (size_t)min(n0 + (col2 & 31), N - 1) * nbr + blk);
+                    st.sc[i] = scale_bits(WF16, col2 & 32 ? ms.s[1] : ms.s[0],
+                                          (size_t)min(swi_row(col2), N - 1) * nbr + blk);
                 else
                     st.sc[i] = scale_bits(WF16, WS, (size_t)min(n0 + col2, N - 1) * nbr + blk);
             }
@@ -189,15 +161,16 @@ __global__ __launch_bounds__(64 * (TM / 32) * (TN / (32 * NJ)) * (4 / CPW), WPE)
         for (int i = 0; i < NSC; i++) {
             const uint32_t sidx = tid + NT * i, blk = sidx % KC;
             if (sidx < KC * TM)
-                sX(buf)[blk * TM + sidx / KC] = u2f(st.sc[i]);
+                sX(buf)[blk * TM + sidx / KC] = scale_value(FMA, st.sc[i]);
             else if (sidx < KC * (TM + TN))
                 sW(buf)[blk * TN + (sidx - KC * TM) / KC] = scale_value(WF16, st.sc[i]);
         }
     };
 
-    float t[CPW][NJ][16];
+    constexpr int NC = ONE ? 1 : CPW;
+    float t[NC][NJ][16];
 #pragma unroll
-    for (int c2 = 0; c2 < CPW; c2++)
+    for (int c2 = 0; c2 < NC; c2++)
 #pragma unroll
         for (int j = 0; j < NJ; j++)
 #pragma unroll
@@ -271,12 +244,19 @@ __global__ __launch_bounds__(64 * (TM / 32) * (TN / (32 * NJ)) * (4 / CPW), WPE)
                 if (m < M && nn1 < N && b1 < nb) dbg[((size_t)m * N + nn1) * nb + b1] = r.d1[v];
             }
         }
-        // dot.rs: t[b & 3] += (sa * sb) * (isum as f32); CS: every block is the chain's
+        // dot.rs: t[b & 3] += (sa * sb) * (isum as f32); CS: every block is the
+        // chain's. quant.rs:276-288: slot = fma(isum as f32, sa * sb, slot)
+        auto add = [](float& o, float p, int d) {
+            if (FMA)
+                o = __builtin_fmaf((float)d, p, o);
+            else
+                o += p * (float)d;
+        };
 #pragma unroll
-        for (int v = 0; v < 16; v++) t[CS ? 0 : c20][j0][v] += r.P[v] * (float)r.d0[v];
+        for (int v = 0; v < 16; v++) add(t[ONE ? 0 : c20][j0][v], r.P[v], r.d0[v]);
         if (b1 < nb) {
 #pragma unroll
-            for (int v = 0; v < 16; v++) t[CS ? 0 : c21][j1][v] += r.P[16 + v] * (float)r.d1[v];
+            for (int v = 0; v < 16; v++) add(t[ONE ? 0 : c21][j1][v], r.P[16 + v], r.d1[v]);
         }
     };
 
@@ -360,14 +340,56 @@ __global__ __launch_bounds__(64 * (TM / 32) * (TN / (32 * NJ)) * (4 / CPW), WPE)
                 if (m < M && n < N) P[(size_t)m * ld + n] = t[0][j][v];
             }
     } else if constexpr (CPW == 4) {
-        // one wave holds all four chains of its outputs
+        // one wave holds its outputs whole: unit j's register v is row 8 (v / 4)
+        // + 4 half + v % 4 of column 32 j + r32
+        auto value = [&](int j, int v) {
+            if constexpr (FMA)
+                return t[0][j][v];
+            else
+                return ((t[0][j][v] + t[1][j][v]) + t[2][j][v]) + t[3][j][v];
+        };
+        auto row = [&](int v) { return m0 + wm0 + 8 * (v >> 2) + 4 * half + (v & 3); };
+        if constexpr ((SWI || ROPE) && NJ == 2) {
+            // the wave's 64 columns: gate and up of a hidden block, or a head's halves
+            const uint32_t at = n0 + (SWI ? wn0 / 2 : wn0);
+            if (at < N) {
 #pragma unroll
-        for (int j = 0; j < NJ; j++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const uint32_t m = m0 + wm0 + 8 * (v >> 2) + 4 * half + (v & 3), n = n0 + wn0 + 32 * j + r32;
-                if (m < M && n < N) Y[(size_t)m * ld + n] = ((t[0][j][v] + t[1][j][v]) + t[2][j][v]) + t[3][j][v];
+                for (int v = 0; v < 16; v++) {
+                    if constexpr (SWI)
+                        swi_out(so, value(0, v), value(1, v), row(v), M, N, at >> 5, r32, etab);
+                    else if (row(v) < M)
+                        rope_out(ro, mi_, Y, ld, value(0, v), value(1, v), row(v), at, r32);
+                }
             }
+        } else if constexpr (SWI || ROPE) {
+            // a wave holds half of that: the tile meets in LDS, a half-wave takes a row
+            constexpr int LDY = TN + 4;
+            static_assert(TM * LDY * 4 <= RING_BYTES, "the tile reuses the ring");
+            float* const sy = (float*)lds;
+#pragma unroll
+            for (int v = 0; v < 16; v++)
+                sy[(wm0 + 8 * (v >> 2) + 4 * half + (v & 3)) * LDY + wn0 + r32] = value(0, v);
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < TM * TN / 2 / NT; k++) {
+                const uint32_t e = (tid + NT * k) >> 5, m = m0 + e / (TN / 64), h = e % (TN / 64);
+                const float* y = sy + (m - m0) * LDY + 64 * h + r32;
+                const uint32_t at = n0 + (SWI ? 32 : 64) * h;
+                if (at >= N) continue;
+                if constexpr (SWI)
+                    swi_out(so, y[0], y[32], m, M, N, at >> 5, r32, etab);
+                else if (m < M)
+                    rope_out(ro, mi_, Y, ld, y[0], y[32], m, at, r32);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    const uint32_t m = row(v), n = n0 + wn0 + 32 * j + r32;
+                    if (m < M && n < N) Y[(size_t)m * ld + n] = value(j, v);
+                }
+        }
     } else {
         // the chains meet in LDS, four consecutive accumulators per lane as
         // one 16-byte store: part[chain][sub][j][v / 4][lane][v % 4]
@@ -392,22 +414,15 @@ __global__ __launch_bounds__(64 * (TM / 32) * (TN / (32 * NJ)) * (4 / CPW), WPE)
             // element e: (sub, v4, lane): rows 8 v4 + 4 (lane / 32) + 0..3 of
             // hidden column n0 + lane % 32, its gate (unit 0) and up (unit 1);
             // the 32 lanes of a half-wave hold one row's Q8 block
-            const uint32_t nbh = N >> 5, pb = so.cm ? cm_block(n0 >> 5, nbh) : n0 >> 5;
 #pragma unroll
             for (int k = 0; k < TM * 8 / NT; k++) {
                 const uint32_t e = tid + NT * k, sb = e >> 8, v4 = (e >> 6) & 3, l = e & 63;
                 const uint32_t og = sb * (WOUT / 4) + v4 * 64 + l;
                 const float4 g4 = sum4(og), u4 = sum4(og + 256);
                 const float gv[4] = {g4.x, g4.y, g4.z, g4.w}, uv[4] = {u4.x, u4.y, u4.z, u4.w};
-                const uint32_t mb = m0 + (sb % SM) * 32 + 8 * v4 + 4 * (l >> 5), col = n0 + (l & 31);
+                const uint32_t mb = m0 + (sb % SM) * 32 + 8 * v4 + 4 * (l >> 5);
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const bool live = mb + r < M;
-                    // cpu.rs:708-710: silu(g) * u
-                    const float h = div_rn(gv[r], 1.0f + glibc_expf(-gv[r], etab)) * uv[r];
-                    const size_t orow = live ? mb + r : 0, oi = orow * N + pb * 32 + (col & 31);
-                    quant_lane(h, live, so.q + oi, so.s + orow * nbh + pb, so.h + orow * nbh + pb);
-                }
+                for (int r = 0; r < 4; r++) swi_out(so, gv[r], uv[r], mb + r, M, N, n0 >> 5, l & 31, etab);
             }
             return;
         }
@@ -420,25 +435,10 @@ __global__ __launch_bounds__(64 * (TM / 32) * (TN / (32 * NJ)) * (4 / CPW), WPE)
                 const uint32_t og = sb * (WOUT / 4) + v4 * 64 + l;
                 const float4 a4 = sum4(og), b4 = sum4(og + 256);
                 const float av[4] = {a4.x, a4.y, a4.z, a4.w}, bv[4] = {b4.x, b4.y, b4.z, b4.w};
-                const uint32_t mb = m0 + (sb % SM) * 32 + 8 * v4 + 4 * (l >> 5), i = l & 31, c0 = n0 + i;
+                const uint32_t mb = m0 + (sb % SM) * 32 + 8 * v4 + 4 * (l >> 5);
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    if (mb + r >= M) continue;
-                    const uint32_t m = mb + r;
-                    if (mi_ == 2) {  // v: to the cache as it is
-                        float* vr = ro.vc + (size_t)ro.slots[m] * ro.kv_dim;
-                        vr[c0] = av[r];
-                        vr[c0 + 32] = bv[r];
-                        continue;
-                    }
-                    // k_rope_kv: r0 = a cos - b sin, r1 = a sin + b cos
-                    const float2 cs = ro.tab[(size_t)ro.pos[m] * 32 + i];
-                    const float r0 = av[r] * cs.x - bv[r] * cs.y;
-                    const float r1 = av[r] * cs.y + bv[r] * cs.x;
-                    float* dst = mi_ == 0 ? Y + (size_t)m * ld : ro.kc + (size_t)ro.slots[m] * ro.kv_dim;
-                    dst[c0] = r0;
-                    dst[c0 + 32] = r1;
-                }
+                for (int r = 0; r < 4; r++)
+                    if (mb + r < M) rope_out(ro, mi_, Y, ld, av[r], bv[r], mb + r, n0, l & 31);
             }
             return;
         }
@@ -489,13 +489,24 @@ static void launch_q8_cs(hipStream_t st, MatSet ms, QuantAct x, size_t rows, siz
                        block, 0, st, ms, x, (uint32_t)rows, (uint32_t)k, mtiles, nullptr, SwiOut{}, RopeOut{});
 }
 
-// The SwiGLU form: one tile per (row block, hidden block of 32).
-template <int TM, int NJ, int CPW, int KC, int NS, int RS, int WPE>
+// The SwiGLU form: TN / 64 hidden blocks of 32 per tile.
+template <int SEM, int TM, int TN, int NJ, int CPW, int KC, int NS, int RS, int WPE>
 static void launch_q8_swi(hipStream_t st, const MatSet& ms, QuantAct x, size_t rows, size_t k, SwiOut so) {
-    const uint32_t mtiles = (uint32_t)((rows + TM - 1) / TM), ntiles = ms.n[0] / 32;
-    const dim3 grid(ntiles * mtiles), block(64 * (TM / 32) * (64 / (32 * NJ)) * (4 / CPW));
-    hipLaunchKernelGGL((k_gemm_q8<SEM_FOUR_PARTIALS_F32, TM, 64, NJ, CPW, KC, NS, RS, WPE, false, true>), grid, block,
-                       0, st, ms, x, (uint32_t)rows, (uint32_t)k, mtiles, nullptr, so, RopeOut{});
+    const uint32_t mtiles = (uint32_t)((rows + TM - 1) / TM), ntiles = (ms.n[0] + TN / 2 - 1) / (TN / 2);
+    const dim3 grid(ntiles * mtiles), block(64 * (TM / 32) * (TN / (32 * NJ)) * (4 / CPW));
+    hipLaunchKernelGGL((k_gemm_q8<SEM, TM, TN, NJ, CPW, KC, NS, RS, WPE, false, true>), grid, block, 0, st, ms, x,
+                       (uint32_t)rows, (uint32_t)k, mtiles, nullptr, so, RopeOut{});
+}
+
+// The q/k/v form with RoPE and kv_write: 64-wide heads.
+template <int SEM, int TM, int TN, int NJ, int CPW, int KC, int NS, int RS, int WPE>
+static void launch_q8_rope(hipStream_t st, MatSet ms, QuantAct x, size_t rows, size_t k, RopeOut ro) {
+    uint32_t total = 0;
+    for (int i = 0; i < 3; i++) ms.tile_end[i] = total += (ms.n[i] + TN - 1) / TN;
+    const uint32_t mtiles = (uint32_t)((rows + TM - 1) / TM);
+    const dim3 grid(total * mtiles), block(64 * (TM / 32) * (TN / (32 * NJ)) * (4 / CPW));
+    hipLaunchKernelGGL((k_gemm_q8<SEM, TM, TN, NJ, CPW, KC, NS, RS, WPE, false, false, false, true>), grid, block, 0,
+                       st, ms, x, (uint32_t)rows, (uint32_t)k, mtiles, nullptr, SwiOut{}, ro);
 }
 
 // The narrow form (few column tiles: o and down at N = 2048), on 16x16x32
@@ -727,8 +738,13 @@ template <int SEM>
 static hipError_t gemm_q8_go(hipStream_t st, const MatSet& ms, size_t k, QuantAct x, size_t rows, int32_t* dbg) {
     // the widest tile that still gives the grid enough workgroups: wider
     // tiles stage fewer bytes per output (A and B rows are shared by more
-    // outputs) but give fewer, longer workgroups
+    // outputs) but give fewer, longer workgroups. Up to two 16x16 units per CU
+    // the direct form, a wave each, is the shortest (2048x2048, 64 rows, 512
+    // units: 7.7 against 8.1 us with 32x32 tiles; at 128 rows 9.4 against 8.4)
     const size_t m128 = (rows + 127) / 128, m64 = (rows + 63) / 64;
+    const bool direct = (rows + 15) / 16 * gemm_col_tiles(ms, 16) <= 512;
+    if (rows < 8 || (direct && m64 * gemm_col_tiles(ms, 64) < 160))
+        return launch_gemm_direct(st, SEM, ms, k, x, rows, dbg);
     if (rows > 64 && m128 * gemm_col_tiles(ms, 64) >= 200)
         launch_q8<SEM, 128, 64, 2, 2, 4, 3, 1, 1>(st, ms, x, rows, k, dbg);
     else if (m64 * gemm_col_tiles(ms, 64) >= 160)
@@ -738,35 +754,62 @@ static hipError_t gemm_q8_go(hipStream_t st, const MatSet& ms, size_t k, QuantAc
     return hipGetLastError();
 }
 
-// Whether the q/k/v GEMM with the RoPE and kv_write epilogue applies: Q8_0,
-// head_dim 64 whole heads, and a row count at which the plain launch takes
-// the 64x64 tiles (the form the epilogue is built in).
-bool qkv_rope_q8_ok(const DevMatrix& q, const DevMatrix& k, const DevMatrix& v, size_t rows) {
-    if (q.storage != KR_STORAGE_Q8_0 || k.storage != KR_STORAGE_Q8_0 || v.storage != KR_STORAGE_Q8_0) return false;
-    if (q.k != k.k || q.k != v.k || k.n != v.n || q.n % 64 != 0 || k.n % 64 != 0 || rows < 8) return false;
-    const size_t tiles = (q.n + k.n + v.n) / 64, m128 = (rows + 127) / 128, m64 = (rows + 63) / 64;
-    return !(rows > 64 && m128 * tiles >= 200) && m64 * tiles >= 160;
+// Q8_0x4: one serial FMA chain per output, so a wave's unit runs over all of K
+// and the launch is as long as one unit where the grid is small (32x32 units in
+// 32x128 tiles: 23 us at 960x2560 for 9 to 700 rows). So the finest unit that
+// the grid allows. Times in us, direct / 64x64 / 128x128, against that form's:
+//   960x960    77 rows  4.8 /  8.4 / 16 (11.1)   700 rows 11.0 /  8.8 / 16 (11.6)
+//   960x2560   77 rows  7.7 / 16.0 / 36 (23.2)   700 rows 23.1 / 16.7 / 36 (23.6)
+//   9216x1536  32 rows 10.8 / 12.0 / 23 (17.0)   128 rows 25.2 / 18.2 / 25 (23.3)
+//   5120x960  700 rows 38.6 / 23.6 / 19 (29.4)  16384x2048, 256 rows 97 / 44 / 37 (59)
+// Direct wins to about 1400 16x16 units, 128x128 from about 640 64x64 tiles.
+static hipError_t gemm_chain_go(hipStream_t st, const MatSet& ms, size_t k, QuantAct x, size_t rows, int32_t* dbg) {
+    if ((rows + 15) / 16 * gemm_col_tiles(ms, 16) <= kDirectTiles16)
+        return launch_gemm_direct(st, SEM_FMA_CHAIN, ms, k, x, rows, dbg);
+    if ((rows + 63) / 64 * gemm_col_tiles(ms, 64) <= kChainTiles64)
+        launch_q8<SEM_FMA_CHAIN, 64, 64, 1, 4, 4, 3, 2, 1>(st, ms, x, rows, k, dbg);
+    else
+        launch_q8<SEM_FMA_CHAIN, 128, 128, 2, 4, 4, 2, 1, 1>(st, ms, x, rows, k, dbg);
+    return hipGetLastError();
 }
 
-hipError_t launch_qkv_rope_q8(hipStream_t st, const DevMatrix& q, const DevMatrix& k, const DevMatrix& v, QuantAct x,
-                              size_t rows, float* yq, const uint32_t* pos, const uint32_t* slots, const float2* tab,
-                              float* kc, float* vc) {
-    if (!qkv_rope_q8_ok(q, k, v, rows)) return hipErrorInvalidValue;
+// Whether the q/k/v GEMM with the RoPE and kv_write epilogue applies: one
+// storage, head_dim 64 whole heads, and for Q8_0 a row count at which the plain
+// launch takes the 64x64 tiles (the form its epilogue is built in) or the
+// direct form's grid.
+static bool qkv_rope_tiles(const DevMatrix& q, const DevMatrix& k, size_t rows) {
+    const size_t tiles = (q.n + 2 * k.n) / 64, m128 = (rows + 127) / 128, m64 = (rows + 63) / 64;
+    return !(rows > 64 && m128 * tiles >= 200) && m64 * tiles >= 160;
+}
+static bool qkv_rope_direct(const DevMatrix& q, const DevMatrix& k, size_t rows) {
+    return (rows + 15) / 16 * ((q.n + 2 * k.n) / 64) <= kDirectRopeMax;
+}
+bool qkv_rope_ok(const DevMatrix& q, const DevMatrix& k, const DevMatrix& v, size_t rows) {
+    if (k.storage != q.storage || v.storage != q.storage) return false;
+    if (q.k != k.k || q.k != v.k || k.n != v.n || q.n % 64 != 0 || k.n % 64 != 0 || rows < 2) return false;
+    return q.storage == KR_STORAGE_Q8_0X4 || qkv_rope_tiles(q, k, rows) || qkv_rope_direct(q, k, rows);
+}
+
+hipError_t launch_qkv_rope(hipStream_t st, const DevMatrix& q, const DevMatrix& k, const DevMatrix& v, QuantAct x,
+                           size_t rows, float* yq, const uint32_t* pos, const uint32_t* slots, const float2* tab,
+                           float* kc, float* vc) {
+    if (!qkv_rope_ok(q, k, v, rows)) return hipErrorInvalidValue;
     MatSet ms{};
     const DevMatrix* w[3] = {&q, &k, &v};
-    uint32_t total = 0;
-    for (int i = 0; i < 3; i++) {
-        ms.q[i] = w[i]->q, ms.s[i] = w[i]->s, ms.n[i] = (uint32_t)w[i]->n;
-        total += (uint32_t)(w[i]->n / 64);
-        ms.tile_end[i] = total;
-    }
+    for (int i = 0; i < 3; i++) ms.q[i] = w[i]->q, ms.s[i] = w[i]->s, ms.n[i] = (uint32_t)w[i]->n;
     ms.y[0] = yq, ms.ld[0] = (uint32_t)q.n;
     ms.count = 3;
     const RopeOut ro{pos, slots, tab, kc, vc, (uint32_t)k.n};
-    const uint32_t mtiles = (uint32_t)((rows + 63) / 64);
-    hipLaunchKernelGGL((k_gemm_q8<SEM_FOUR_PARTIALS_F32, 64, 64, 2, 1, 8, 2, 2, 1, false, false, false, true>),
-                       dim3(total * mtiles), dim3(64 * 2 * 1 * 4), 0, st, ms, x, (uint32_t)rows, (uint32_t)q.k, mtiles,
-                       nullptr, SwiOut{}, ro);
+    if (q.storage == KR_STORAGE_Q8_0X4) {
+        if (qkv_rope_direct(q, k, rows)) return launch_direct_rope(st, SEM_FMA_CHAIN, ms, q.k, x, rows, ro);
+        if ((rows + 63) / 64 * ((q.n + 2 * k.n) / 64) <= kChainTiles64)
+            launch_q8_rope<SEM_FMA_CHAIN, 64, 64, 1, 4, 4, 3, 2, 1>(st, ms, x, rows, q.k, ro);
+        else
+            launch_q8_rope<SEM_FMA_CHAIN, 128, 128, 2, 4, 4, 2, 1, 1>(st, ms, x, rows, q.k, ro);
+        return hipGetLastError();
+    }
+    if (!qkv_rope_tiles(q, k, rows)) return launch_direct_rope(st, SEM_FOUR_PARTIALS_F32, ms, q.k, x, rows, ro);
+    launch_q8_rope<SEM_FOUR_PARTIALS_F32, 64, 64, 2, 1, 8, 2, 2, 1>(st, ms, x, rows, q.k, ro);
     return hipGetLastError();
 }
 
@@ -792,10 +835,10 @@ hipError_t launch_mfma_f32_probe(hipStream_t st, const float* a, const float* b,
     return hipGetLastError();
 }
 
-hipError_t launch_gate_up_silu_q8(hipStream_t st, const DevMatrix& gate, const DevMatrix& up, QuantAct x, size_t rows,
-                                  int8_t* hq, float* hs, uint16_t* hh, bool chain_major) {
-    if (gate.storage != KR_STORAGE_Q8_0 || up.storage != KR_STORAGE_Q8_0 || gate.n != up.n || gate.k != up.k ||
-        gate.n % 32 != 0 || rows == 0 || (chain_major && gate.n % 128 != 0))
+hipError_t launch_gate_up_silu(hipStream_t st, const DevMatrix& gate, const DevMatrix& up, QuantAct x, size_t rows,
+                               int8_t* hq, float* hs, uint16_t* hh, bool chain_major) {
+    if (gate.storage != up.storage || gate.n != up.n || gate.k != up.k || gate.n % 32 != 0 || rows == 0 ||
+        (chain_major && gate.n % 128 != 0))
         return hipErrorInvalidValue;
     MatSet ms{};
     ms.q[0] = gate.q, ms.q[1] = up.q;
@@ -803,11 +846,20 @@ hipError_t launch_gate_up_silu_q8(hipStream_t st, const DevMatrix& gate, const D
     ms.n[0] = ms.n[1] = (uint32_t)gate.n;
     ms.count = 2;
     const SwiOut so{hq, hs, hh, chain_major ? 1u : 0u};
-    const size_t m128 = (rows + 127) / 128, blocks = gate.n / 32;
+    const size_t m128 = (rows + 127) / 128, blocks = gate.n / 32, direct = (rows + 15) / 16 * blocks;
+    if (gate.storage == KR_STORAGE_Q8_0X4) {
+        if (direct <= kDirectSwiMax) return launch_direct_swi(st, SEM_FMA_CHAIN, ms, gate.k, x, rows, so);
+        if ((rows + 63) / 64 * blocks <= kChainTiles64)
+            launch_q8_swi<SEM_FMA_CHAIN, 64, 64, 1, 4, 4, 3, 2, 1>(st, ms, x, rows, gate.k, so);
+        else
+            launch_q8_swi<SEM_FMA_CHAIN, 128, 128, 2, 4, 4, 2, 1, 1>(st, ms, x, rows, gate.k, so);
+        return hipGetLastError();
+    }
+    if (rows < 8) return launch_direct_swi(st, SEM_FOUR_PARTIALS_F32, ms, gate.k, x, rows, so);
     if (rows > 64 && m128 * blocks >= 200)
-        launch_q8_swi<128, 2, 2, 4, 3, 1, 1>(st, ms, x, rows, gate.k, so);
+        launch_q8_swi<SEM_FOUR_PARTIALS_F32, 128, 64, 2, 2, 4, 3, 1, 1>(st, ms, x, rows, gate.k, so);
     else
-        launch_q8_swi<64, 2, 1, 8, 2, 2, 1>(st, ms, x, rows, gate.k, so);
+        launch_q8_swi<SEM_FOUR_PARTIALS_F32, 64, 64, 2, 1, 8, 2, 2, 1>(st, ms, x, rows, gate.k, so);
     return hipGetLastError();
 }
 
@@ -845,6 +897,7 @@ hipError_t launch_gemm_q8_cs(hipStream_t st, const DevMatrix& cm, QuantAct x, si
 
 hipError_t launch_gemm_q8(hipStream_t st, int sem, const MatSet& ms, size_t k, QuantAct x, size_t rows,
                           int32_t* dbg) {
+    if (sem == SEM_FMA_CHAIN) return gemm_chain_go(st, ms, k, x, rows, dbg);
     if (sem == SEM_FOUR_PARTIALS_F32) return gemm_q8_go<SEM_FOUR_PARTIALS_F32>(st, ms, k, x, rows, dbg);
     if (sem == SEM_FOUR_PARTIALS_F16) return gemm_q8_go<SEM_FOUR_PARTIALS_F16>(st, ms, k, x, rows, dbg);
     return hipErrorInvalidValue;

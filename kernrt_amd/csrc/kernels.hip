@@ -1158,183 +1158,20 @@ bool swiglu_fusable(const DevMatrix& gate, const DevMatrix& up) {
 }
 
 // ---------------------------------------------------------------------------
-// Quantized GEMM on int8 MFMA (prefill and batched rows, M >= kGemmMinRows).
-// The four-partial Q8_0 GEMM (dot.rs:35-44) is k_gemm_q8 in gemm.hip; this
-// file holds the Q8_0x4 FMA chain (quant.rs:276-288, k_gemm_chain).
-//
-// v_mfma_i32_32x32x32_i8 multiplies a 32x32 int8 tile of activations by a
-// 32x32 int8 tile of weights over K = 32, exactly one Q8 block, so each
-// instruction yields the exact i32 block dots of a 32x32 output tile. Every
-// block's dots go straight into the reference's f32 epilogue, so each output
-// keeps the per-row path's rounding sequence.
-//
-// Operand layout: lane l feeds row l % 32 of the activation tile and column
-// l % 32 of the weight tile with bytes 16*(l/32) .. +16 of the block; both
-// operands use the same byte map, so the integer sum covers the block once.
-// Accumulator v of lane l is output (row 8*(v/4) + 4*(l/32) + v%4, col l%32).
-//
-// The chain is serial, so each wave owns its own 32x32 tile over all of K;
-// the workgroup tile is 32x128 and the 4 waves share the activation chunk.
-// Operands are staged through LDS in chunks of KC = 4 blocks: every row's
-// KC*32 bytes are read with coalesced 16-byte loads (whole cache lines),
-// several chunks ahead in registers, and written to a double-buffered LDS
-// tile whose rows are padded by 16 bytes so that the fragment reads of 32
-// consecutive rows spread over all banks. One barrier per chunk.
-//
-// Workgroups are numbered XCD-aware: the row tiles that share a column tile
-// of weights run on one XCD and share its L2.
-typedef int v16i __attribute__((ext_vector_type(16)));
-static constexpr size_t kGemmMinRows = 8;
-// chunks each thread keeps in flight in registers (even: LDS buffer parity)
-static constexpr int kGemmStages = 4;
-
-// Workgroup ids are dispatched round-robin over the 8 XCDs; map them so that
-// consecutive logical tiles run on one XCD.
-__device__ __forceinline__ uint32_t xcd_tile(uint32_t id, uint32_t count) {
-    const uint32_t per = count >> 3, rem = count & 7, xcd = id & 7, k = id >> 3;
-    return xcd < rem ? xcd * (per + 1) + k : rem * (per + 1) + (xcd - rem) * per + k;
-}
-
-// One column tile of a matrix in the set; tile_end counts column tiles of
-// width `cols`.
-struct GemmPos {
-    int mi;
-    uint32_t m0, n0;
-};
-__device__ __forceinline__ GemmPos gemm_pos(const MatSet& ms, uint32_t mtiles, uint32_t cols) {
-    const uint32_t L = xcd_tile(blockIdx.x, gridDim.x);
-    const uint32_t mt = L % mtiles, nt = L / mtiles;
-    const int mi = nt < ms.tile_end[0] ? 0 : (nt < ms.tile_end[1] ? 1 : 2);
-    const uint32_t tile = nt - (mi == 0 ? 0 : ms.tile_end[mi - 1]);
-    return GemmPos{mi, mt * 32, tile * cols};
-}
-
-// The 16 activation scales of accumulator rows 8g + 4*half + (0..3).
-__device__ __forceinline__ void gemm_row_scales(float (&xs)[16], const float* col) {
-    const float4* q = (const float4*)col;
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-        const float4 f = q[2 * g];
-        xs[4 * g] = f.x, xs[4 * g + 1] = f.y, xs[4 * g + 2] = f.z, xs[4 * g + 3] = f.w;
-    }
-}
-
-template <bool DBG>
-__global__ __launch_bounds__(256, 2) void k_gemm_chain(MatSet ms, QuantAct x, uint32_t M, uint32_t K,
-                                                       uint32_t mtiles, int32_t* __restrict__ dbg) {
-    constexpr int KC = 4, ROW = KC * 32 + 16, NS = kGemmStages;
-    __shared__ __align__(16) int8_t sA[2][32 * ROW];
-    __shared__ __align__(16) int8_t sB[2][128 * ROW];
-    __shared__ __align__(16) float sX[2][KC * 32];   // [block][row]
-    __shared__ __align__(16) float sW[2][KC * 128];  // [block][col]
-    const uint32_t nb = K >> 5, nchunks = (nb + KC - 1) / KC;
-    const GemmPos p = gemm_pos(ms, mtiles, 128);
-    const int8_t* __restrict__ W = ms.q[p.mi];
-    const uint16_t* __restrict__ WS = (const uint16_t*)ms.s[p.mi];
-    const uint32_t N = ms.n[p.mi];
-    const uint32_t tid = threadIdx.x, lane = tid & 63;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: block checks branch on SGPRs
-    const uint32_t r = lane & 31, half = lane >> 5;
-    const uint32_t n = p.n0 + 32 * wave + r;       // this lane's output column
-    const bool active = p.n0 + 32 * wave < N;       // uniform per wave
-
-    // loader map: activation piece (row tid/8, 16-byte column tid%8), weight
-    // pieces (rows tid/8 + 32i), activation scale (row (tid/4)%32, block
-    // tid%4; the upper half of the workgroup repeats the lower), weight
-    // scales (columns tid/4 + 64i, block tid%4).
-    const uint32_t lr = tid >> 3, lc = (tid & 7) * 16, xr = (tid >> 2) & 31, wc = tid >> 2, sb = tid & 3;
-    const int8_t* ga = x.q + (size_t)min(p.m0 + lr, M - 1) * K;
-    const int8_t* gb[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) gb[i] = W + (size_t)min(p.n0 + lr + 32 * i, N - 1) * K;
-    const uint16_t* gx = x.h + (size_t)min(p.m0 + xr, M - 1) * nb;
-    const size_t gw0 = (size_t)min(p.n0 + wc, N - 1) * nb, gw1 = (size_t)min(p.n0 + wc + 64, N - 1) * nb;
-
-    struct Stage {
-        v4i a, b[4];
-        uint32_t xs, w0, w1;
-    };
-    auto gload = [&](Stage& st, uint32_t c) {
-        c = c < nchunks ? c : nchunks - 1;
-        const uint32_t col = min(c * KC * 32 + lc, K - 16);  // past the row end: a piece no block uses
-        st.a = *(const v4i*)(ga + col);
-#pragma unroll
-        for (int i = 0; i < 4; i++) st.b[i] = *(const v4i*)(gb[i] + col);
-        const uint32_t blk = min(c * KC + sb, nb - 1);
-        st.xs = gx[blk];
-        st.w0 = WS[gw0 + blk], st.w1 = WS[gw1 + blk];
-    };
-    auto lstore = [&](const Stage& st, int buf) {
-        *(v4i*)(sA[buf] + lr * ROW + lc) = st.a;
-#pragma unroll
-        for (int i = 0; i < 4; i++) *(v4i*)(sB[buf] + (lr + 32 * i) * ROW + lc) = st.b[i];
-        sX[buf][sb * 32 + xr] = f16w((uint16_t)st.xs);
-        sW[buf][sb * 128 + wc] = f16w((uint16_t)st.w0);
-        sW[buf][sb * 128 + wc + 64] = f16w((uint16_t)st.w1);
-    };
-
-    const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    float slot[16];
-#pragma unroll
-    for (int v = 0; v < 16; v++) slot[v] = 0.0f;
-    auto compute = [&](int buf, uint32_t c) {
-        if (!active) return;
-#pragma unroll
-        for (int blk = 0; blk < KC; blk++) {
-            const uint32_t b = c * KC + blk;
-            if (b >= nb) break;
-            const v4i a = *(const v4i*)(sA[buf] + r * ROW + blk * 32 + 16 * half);
-            const v4i bq = *(const v4i*)(sB[buf] + (32 * wave + r) * ROW + blk * 32 + 16 * half);
-            const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, bq, zero, 0, 0, 0);
-            const float w = sW[buf][blk * 128 + 32 * wave + r];
-            float xs[16];
-            gemm_row_scales(xs, sX[buf] + blk * 32 + 4 * half);
-            if (DBG && n < N) {
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const uint32_t m = p.m0 + 8 * (v >> 2) + 4 * half + (v & 3);
-                    if (m < M) dbg[((size_t)m * N + n) * nb + b] = d[v];
-                }
-            }
-            // quant.rs: slot = (isum as f32).mul_add(f16w(ws) * f16w(xs), slot)
-#pragma unroll
-            for (int v = 0; v < 16; v++) slot[v] = __builtin_fmaf((float)d[v], w * xs[v], slot[v]);
-        }
-    };
-
-    gemm_pipeline<NS, Stage>(nchunks, gload, lstore, compute);
-    if (!active || n >= N) return;
-    float* Y = ms.y[p.mi];
-    const uint32_t ld = ms.ld[p.mi];
-#pragma unroll
-    for (int v = 0; v < 16; v++) {
-        const uint32_t m = p.m0 + 8 * (v >> 2) + 4 * half + (v & 3);
-        if (m < M) Y[(size_t)m * ld + n] = slot[v];
-    }
-}
-
-template <int SEM>
-static hipError_t gemm_launch(hipStream_t st, MatSet ms, size_t k, QuantAct x, size_t rows, int32_t* dbg) {
-    if (SEM != SEM_FMA_CHAIN) return launch_gemm_q8(st, SEM, ms, k, x, rows, dbg);
-    const uint32_t cols = 128;
-    uint32_t total = 0;
-    for (int i = 0; i < 3; i++) {
-        if (i < ms.count) total += (uint32_t)((ms.n[i] + cols - 1) / cols);
-        ms.tile_end[i] = total;
-    }
-    const uint32_t mtiles = (uint32_t)((rows + 31) / 32);
-    dim3 grid(total * mtiles);
-    const uint32_t m = (uint32_t)rows, kk = (uint32_t)k;
-    if (dbg)
-        hipLaunchKernelGGL(k_gemm_chain<true>, grid, dim3(256), 0, st, ms, x, m, kk, mtiles, dbg);
-    else
-        hipLaunchKernelGGL(k_gemm_chain<false>, grid, dim3(256), 0, st, ms, x, m, kk, mtiles, dbg);
-    return hipGetLastError();
+// From how many rows on a projection takes the matrix core (gemm.hip). The GEMV
+// serves four rows per pass over the weights, so five to seven rows cost two
+// passes: 960x2560 Q8_0x4, 6 rows, 9.1 against 7.3 us direct; 5120x960 9.7
+// against 5.2. With the four partial sums the direct form needs a wide output to
+// win (4096x1024 7.9 against 5.5 us, but 1024x2048 6.2 against 6.9).
+static size_t gemm_min_rows(int sem, const MatSet& ms) {
+    size_t n = 0;
+    for (int i = 0; i < ms.count; i++) n += ms.n[i];
+    return sem == SEM_FMA_CHAIN || n >= 3200 ? 5 : 8;
 }
 
 template <int SEM>
 static hipError_t gemv_rows(hipStream_t st, const MatSet& ms, size_t k, QuantAct x, size_t rows, int32_t* dbg) {
-    if (rows >= kGemmMinRows) return gemm_launch<SEM>(st, ms, k, x, rows, dbg);
+    if (rows >= gemm_min_rows(SEM, ms)) return launch_gemm_q8(st, SEM, ms, k, x, rows, dbg);
     size_t nb = k / 32;
     size_t done = 0;
     while (done < rows) {
@@ -4182,6 +4019,7 @@ __global__ __launch_bounds__(256) void k_mfma_spin(int* __restrict__ sink, uint3
     int s = 0;
     if (KIND == 0) {
         const v4i a = {t, t + 1, t + 2, t + 3}, b = {3 * t, t ^ 5, t + 7, 1};
+        typedef int v16i __attribute__((ext_vector_type(16)));
         v16i acc[4] = {};
         for (uint32_t i = 0; i < iters; i++)
 #pragma unroll
