@@ -41,15 +41,16 @@ struct MxBlock {
     DevWindow w0;
 };
 template <int G>
-__device__ __forceinline__ MxBlock mx_block(const DevWindow* windows, uint32_t n_rows, uint32_t kv_mul, uint32_t hs,
-                                            uint32_t* s_cnt) {
+__device__ __forceinline__ MxBlock mx_block(const DevWindow* windows, const uint32_t* blocks, uint32_t n_rows,
+                                            uint32_t kv_mul, uint32_t hs, uint32_t* s_cnt) {
     constexpr uint32_t R = 32 / G;
     MxBlock b;
     // the last row blocks first: a causal prefill's windows grow with the
     // row, so the longest blocks start first and the short ones fill in
     // behind them, instead of leaving the long ones for the tail
-    b.r0 = (gridDim.y - 1 - blockIdx.y) * R;
-    b.nr = min(R, n_rows - b.r0);
+    const uint32_t bi = gridDim.y - 1 - blockIdx.y;
+    b.r0 = blocks ? blocks[bi] : bi * R;
+    b.nr = blocks ? blocks[bi + 1] - b.r0 : min(R, n_rows - b.r0);
     b.h0 = blockIdx.x * G;
     b.kvo = (b.h0 / kv_mul) * hs;
     b.w0 = windows[b.r0];
@@ -69,7 +70,8 @@ __global__ __launch_bounds__(256) void k_attn_mx_scores(const float* __restrict_
                                                         const float* __restrict__ kc, size_t loff,
                                                         const DevWindow* __restrict__ windows, uint32_t n_rows,
                                                         uint32_t n_heads, uint32_t kv_mul, uint32_t kv_dim,
-                                                        uint32_t seq_len, float scale, float* __restrict__ pmax) {
+                                                        uint32_t seq_len, float scale, float* __restrict__ pmax,
+                                                        const uint32_t* __restrict__ blocks) {
     constexpr uint32_t NS = HS / 4, KCH = 8, QST = HS + 4;
     static_assert(32 % G == 0 && (HS == 64 || HS == 128) && NS % KCH == 0, "shape");
     __shared__ __align__(16) float s_q[32 * QST];  // the pairs' q rows
@@ -82,7 +84,7 @@ __global__ __launch_bounds__(256) void k_attn_mx_scores(const float* __restrict_
     const uint32_t tid = threadIdx.x, lane = tid & 63, h = lane >> 5, pr = lane & 31;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t width = n_heads * HS;
-    const MxBlock B = mx_block<G>(windows, n_rows, kv_mul, HS, s_cnt);
+    const MxBlock B = mx_block<G>(windows, blocks, n_rows, kv_mul, HS, s_cnt);
     const uint32_t r0 = B.r0, nr = B.nr, h0 = B.h0, n_shared = B.n_shared, cmax = B.cmax;
     const DevWindow w0 = B.w0;
     // q rows of the 32 pairs (pairs past the block read the last one)
@@ -295,7 +297,7 @@ __global__ __launch_bounds__(256, 3) void k_attn_mx_v(float* __restrict__ att, f
                                                    uint32_t n_heads, uint32_t kv_mul, uint32_t kv_dim,
                                                    uint32_t seq_len, int8_t* __restrict__ qo, float* __restrict__ so,
                                                    uint16_t* __restrict__ ho, const float* __restrict__ psum,
-                                                   uint32_t keep_att) {
+                                                   uint32_t keep_att, const uint32_t* __restrict__ blocks) {
     constexpr uint32_t VST = HS + 4, PST = 33;
     static_assert(32 % G == 0 && (HS == 64 || HS == 128), "shape");
     __shared__ __align__(16) float s_v[2][32 * VST];  // V chunk [position][dim]
@@ -304,7 +306,7 @@ __global__ __launch_bounds__(256, 3) void k_attn_mx_v(float* __restrict__ att, f
     const uint32_t tid = threadIdx.x, lane = tid & 63, h = lane >> 5, pr = lane & 31;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t width = n_heads * HS;
-    const MxBlock B = mx_block<G>(windows, n_rows, kv_mul, HS, s_cnt);
+    const MxBlock B = mx_block<G>(windows, blocks, n_rows, kv_mul, HS, s_cnt);
     const uint32_t r0 = B.r0, nr = B.nr, h0 = B.h0, n_shared = B.n_shared, cmax = B.cmax;
     const DevWindow w0 = B.w0;
     const float* vbase = vc + loff + B.kvo;
@@ -474,46 +476,39 @@ static constexpr size_t kAttnMxMinWindow128 = 160, kAttnMxMinWindow64 = 768;
 // third of the rate)
 static constexpr size_t kAttnMxMaxWindow = 16384;
 // k_attn_mx: query heads per workgroup (the largest of 8, 4, 2, 1 dividing
-// kv_mul), and whether a launch can take it: head size 64 or 128, windows
-// of at most kAttnMxMaxWindow positions, n_rows >= 2 and every block of 32 / G rows
-// sharing one window layout (prefill).
+// kv_mul), and the rows of its blocks, which share one window layout (prefill):
+// head size 64 or 128, a longest window of at most kAttnMxMaxWindow positions.
 static size_t attn_mx_group(size_t kv_mul) {
     for (size_t g : {8, 4, 2})
         if (kv_mul % g == 0) return g;
     return 1;
 }
-bool attention_mx_ok(const DevWindow* w, size_t n_rows, size_t max_count, size_t kv_mul, size_t hs) {
+size_t attention_mx_rows(size_t max_count, size_t kv_mul, size_t hs) {
     // shorter windows run faster on k_attn_rows (one launch, more workgroups)
     const size_t min_window = hs == 128 ? kAttnMxMinWindow128 : kAttnMxMinWindow64;
-    if ((hs != 64 && hs != 128) || max_count < min_window || max_count > kAttnMxMaxWindow || n_rows < 2) return false;
-    const size_t R = 32 / attn_mx_group(kv_mul);
-    for (size_t r = 0; r < n_rows; r++) {
-        const DevWindow& a = w[r - r % R];
-        if (a.att_start != w[r].att_start || a.shared_start != w[r].shared_start || a.shared_end != w[r].shared_end)
-            return false;
-    }
-    return true;
+    if ((hs != 64 && hs != 128) || max_count < min_window || max_count > kAttnMxMaxWindow) return 0;
+    return 32 / attn_mx_group(kv_mul);
 }
 
 hipError_t launch_attention_mx(hipStream_t st, const float* q, float* out, float* att, const float* kc,
                                const float* vc, size_t layer, const DevWindow* windows, size_t n_rows,
                                size_t max_count, size_t n_heads, size_t kv_mul, size_t hs, size_t kv_dim,
                                size_t seq_len, float scale, int8_t* qo, float* so, uint16_t* ho, float* scratch,
-                               bool keep_att) {
+                               bool keep_att, const uint32_t* blocks, size_t n_blocks) {
     const size_t G = attn_mx_group(kv_mul), R = 32 / G;
-    const dim3 grid((unsigned)(n_heads / G), (unsigned)((n_rows + R - 1) / R));
+    const dim3 grid((unsigned)(n_heads / G), (unsigned)(blocks ? n_blocks : (n_rows + R - 1) / R));
     const dim3 gsm((unsigned)((n_rows * n_heads + kMxSmPairs - 1) / kMxSmPairs));
     float* pmax = scratch;                  // each pair's max
     float* psum = scratch + n_rows * n_heads;  // and its sum of exps
 #define KR_ATTN_MX(g, h)                                                                                         \
     hipLaunchKernelGGL((k_attn_mx_scores<g, h>), grid, dim3(256), 0, st, q, att, kc, layer * seq_len * kv_dim,      \
                        windows, (uint32_t)n_rows, (uint32_t)n_heads, (uint32_t)kv_mul, (uint32_t)kv_dim,           \
-                       (uint32_t)seq_len, scale, pmax);                                                            \
+                       (uint32_t)seq_len, scale, pmax, blocks);                                                            \
     hipLaunchKernelGGL(k_attn_softmax_att, gsm, dim3(256), 0, st, att, windows, (uint32_t)n_rows, (uint32_t)n_heads, \
                        (uint32_t)seq_len, pmax, psum);                                                             \
     hipLaunchKernelGGL((k_attn_mx_v<g, h>), grid, dim3(256), 0, st, att, out, vc, layer * seq_len * kv_dim, windows, \
                        (uint32_t)n_rows, (uint32_t)n_heads, (uint32_t)kv_mul, (uint32_t)kv_dim, (uint32_t)seq_len, \
-                       qo, so, ho, psum, keep_att ? 1u : 0u)
+                       qo, so, ho, psum, keep_att ? 1u : 0u, blocks)
 #define KR_ATTN_MX_G(g)     \
     if (hs == 64) {         \
         KR_ATTN_MX(g, 64);  \

@@ -900,21 +900,46 @@ int ensure_attn_scratch(kr_ctx* c, size_t need) {
     return KR_OK;
 }
 
-// Attention over n >= 1 rows with host windows `w` (staged at `wd`): rows
-// whose windows differ (batched decode of separate sequences) take the
-// two-launch split form, everything else launch_attention.
-int attention_many(kr_ctx* c, const float* q, float* out, float* att, size_t layer, const uint32_t* wd,
-                   const std::vector<uint32_t>& w, size_t n, size_t max_count, const kr_attn_spec* sp,
-                   int8_t* qo, float* so, uint16_t* ho, bool keep_att = true) {
-    const kr::DevWindow* hw = (const kr::DevWindow*)w.data();
+// The n >= 1 windows of an attention call checked, the launches they take
+// chosen, and both in device memory: the windows, then the plan's blocks.
+struct StagedWindows {
+    const uint32_t* dev = nullptr;
+    size_t max_count = 0;
+    kr::AttnPlan plan;
+};
+int stage_windows(kr_ctx* c, const kr_window* windows, size_t n, const kr_attn_spec* sp, StagedWindows* out) {
+    std::vector<uint32_t> w(4 * n);
+    for (size_t i = 0; i < n; i++) {
+        const kr_window& x = windows[i];
+        CHECK(c, x.att_start <= x.slot && x.slot < c->seq_len && x.shared_start <= x.shared_end &&
+                     x.shared_end <= c->seq_len,
+              "window %zu out of range", i);
+        const size_t count = (x.shared_end - x.shared_start) + x.slot - x.att_start + 1;
+        CHECK(c, count <= c->seq_len, "window %zu attends more than seq_len slots", i);
+        out->max_count = std::max(out->max_count, count);
+        w[4 * i] = (uint32_t)x.att_start;
+        w[4 * i + 1] = (uint32_t)x.slot;
+        w[4 * i + 2] = (uint32_t)x.shared_start;
+        w[4 * i + 3] = (uint32_t)x.shared_end;
+    }
+    out->plan = kr::attention_plan((const kr::DevWindow*)w.data(), n, out->max_count, sp->n_heads, sp->kv_mul,
+                                   sp->head_size);
+    w.insert(w.end(), out->plan.blocks.begin(), out->plan.blocks.end());
+    return stage(c, c->st_win, w.data(), w.size(), &out->dev);
+}
+
+// Attention over n >= 1 rows by the plan of their staged windows.
+int attention_many(kr_ctx* c, const float* q, float* out, float* att, size_t layer, const StagedWindows& w, size_t n,
+                   const kr_attn_spec* sp, int8_t* qo, float* so, uint16_t* ho, bool keep_att = true) {
+    const kr::DevWindow* wd = (const kr::DevWindow*)w.dev;
     const float scale = 1.0f / sqrtf((float)sp->head_size);  // cpu.rs:591
-    if (n >= 2 && !kr::attention_rows_uniform(hw, n, max_count, sp->kv_mul, sp->head_size) &&
-        kr::attention_split_rows_ok(max_count, sp->kv_mul, sp->head_size)) {
-        int rc = ensure_attn_scratch(c, n * kr::attention_split_scratch(sp->n_heads, c->seq_len));
+    if (w.plan.kind == kr::ATTN_SPLIT) {
+        int rc = ensure_attn_scratch(
+            c, n * kr::attention_split_scratch(sp->n_heads, kr::attention_split_cap(w.max_count, c->seq_len)));
         if (rc) return rc;
-        HIPCHK(c, kr::launch_attention_split_rows(c->stream, q, out, att, c->kc, c->vc, layer, (const kr::DevWindow*)wd,
-                                                  n, max_count, sp->n_heads, sp->kv_mul, sp->head_size, sp->kv_dim,
-                                                  sp->seq_len, scale, c->attn_scratch, keep_att,
+        HIPCHK(c, kr::launch_attention_split_rows(c->stream, q, out, att, c->kc, c->vc, layer, wd, n, w.max_count,
+                                                  sp->n_heads, sp->kv_mul, sp->head_size, sp->kv_dim, sp->seq_len,
+                                                  scale, c->attn_scratch, keep_att,
                                                   sp->head_size % 32 == 0 ? qo : nullptr, so, ho));
         const size_t width = sp->n_heads * sp->head_size;
         if (qo && sp->head_size % 32 != 0) HIPCHK(c, kr::launch_quantize(c->stream, out, n, width, width, qo, so, ho));
@@ -923,9 +948,9 @@ int attention_many(kr_ctx* c, const float* q, float* out, float* att, size_t lay
     // the matrix-core prefill attention keeps each pair's max and sum in the scratch
     int rc = ensure_attn_scratch(c, 2 * n * sp->n_heads);
     if (rc) return rc;
-    HIPCHK(c, kr::launch_attention(c->stream, q, out, att, c->kc, c->vc, layer, (const kr::DevWindow*)wd, n, max_count,
-                                   sp->n_heads, sp->kv_mul, sp->head_size, sp->kv_dim, sp->seq_len, scale, qo, so, ho,
-                                   hw, c->attn_scratch, keep_att));
+    HIPCHK(c, kr::launch_attention(c->stream, q, out, att, c->kc, c->vc, layer, wd, n, w.max_count, sp->n_heads,
+                                   sp->kv_mul, sp->head_size, sp->kv_dim, sp->seq_len, scale, qo, so, ho, w.plan,
+                                   w.dev + 4 * n, c->attn_scratch, keep_att));
     return KR_OK;
 }
 
@@ -944,25 +969,10 @@ int kr_attention(kr_ctx* c, kr_buf q, kr_buf out, kr_buf att, size_t layer, cons
     BUF(ob, out, n * width);
     BUF(ab, att, n * sp->n_heads * sp->seq_len);
     if (n == 0) return KR_OK;
-    std::vector<uint32_t> w(4 * n);
-    size_t max_count = 0;
-    for (size_t i = 0; i < n; i++) {
-        const kr_window& x = windows[i];
-        CHECK(c, x.att_start <= x.slot && x.slot < c->seq_len && x.shared_start <= x.shared_end &&
-                     x.shared_end <= c->seq_len,
-              "window %zu out of range", i);
-        size_t count = (x.shared_end - x.shared_start) + x.slot - x.att_start + 1;
-        CHECK(c, count <= c->seq_len, "window %zu attends more than seq_len slots", i);
-        max_count = count > max_count ? count : max_count;
-        w[4 * i] = (uint32_t)x.att_start;
-        w[4 * i + 1] = (uint32_t)x.slot;
-        w[4 * i + 2] = (uint32_t)x.shared_start;
-        w[4 * i + 3] = (uint32_t)x.shared_end;
-    }
-    const uint32_t* wd;
-    int rc = stage(c, c->st_win, w.data(), 4 * n, &wd);
+    StagedWindows w;
+    int rc = stage_windows(c, windows, n, sp, &w);
     if (rc) return rc;
-    return attention_many(c, qb->p, ob->p, ab->p, layer, wd, w, n, max_count, sp, nullptr, nullptr, nullptr);
+    return attention_many(c, qb->p, ob->p, ab->p, layer, w, n, sp, nullptr, nullptr, nullptr);
 }
 
 int kr_add_in_place(kr_ctx* c, kr_buf dst, kr_buf src, size_t len) {
@@ -1619,41 +1629,19 @@ int attention_quant(kr_ctx* c, kr_buf q, kr_buf out, kr_buf att, size_t layer, c
     BUF(ob, out, n * width);
     BUF(ab, att, n * sp->n_heads * sp->seq_len);
     if (n == 0) return KR_OK;
-    const uint32_t* wd;
-    size_t max_count;
-    std::vector<uint32_t> w;  // host copy of the windows, read by launch_attention
-    if (window_dev) {
-        CHECK(c, n == 1, "a device window is for one row");
-        wd = window_dev;
-        max_count = c->seq_len;
-    } else {
-        w.resize(4 * n);
-        max_count = 0;
-        for (size_t i = 0; i < n; i++) {
-            const kr_window& x = windows[i];
-            CHECK(c, x.att_start <= x.slot && x.slot < c->seq_len && x.shared_start <= x.shared_end &&
-                         x.shared_end <= c->seq_len,
-                  "window %zu out of range", i);
-            size_t count = (x.shared_end - x.shared_start) + x.slot - x.att_start + 1;
-            CHECK(c, count <= c->seq_len, "window %zu attends more than seq_len slots", i);
-            max_count = count > max_count ? count : max_count;
-            w[4 * i] = (uint32_t)x.att_start;
-            w[4 * i + 1] = (uint32_t)x.slot;
-            w[4 * i + 2] = (uint32_t)x.shared_start;
-            w[4 * i + 3] = (uint32_t)x.shared_end;
-        }
-        int rc = stage(c, c->st_win, w.data(), 4 * n, &wd);
-        if (rc) return rc;
-    }
     int rc = ensure_workspace(c, n, width);
     if (rc) return rc;
-    if (w.empty()) {  // one device window
+    if (window_dev) {
+        CHECK(c, n == 1, "a device window is for one row");
         float scale = 1.0f / sqrtf((float)sp->head_size);
-        HIPCHK(c, kr::launch_attention(c->stream, qb->p, ob->p, ab->p, c->kc, c->vc, layer, (const kr::DevWindow*)wd,
-                                       n, max_count, sp->n_heads, sp->kv_mul, sp->head_size, sp->kv_dim, sp->seq_len,
-                                       scale, c->wq, c->ws, c->wh));
+        HIPCHK(c, kr::launch_attention(c->stream, qb->p, ob->p, ab->p, c->kc, c->vc, layer,
+                                       (const kr::DevWindow*)window_dev, n, c->seq_len, sp->n_heads, sp->kv_mul,
+                                       sp->head_size, sp->kv_dim, sp->seq_len, scale, c->wq, c->ws, c->wh));
     } else {
-        rc = attention_many(c, qb->p, ob->p, ab->p, layer, wd, w, n, max_count, sp, c->wq, c->ws, c->wh, keep_att);
+        StagedWindows w;
+        rc = stage_windows(c, windows, n, sp, &w);
+        if (rc) return rc;
+        rc = attention_many(c, qb->p, ob->p, ab->p, layer, w, n, sp, c->wq, c->ws, c->wh, keep_att);
         if (rc) return rc;
     }
     c->q_rows = n;

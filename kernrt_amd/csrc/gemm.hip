@@ -767,7 +767,7 @@ static hipError_t gemm_chain_go(hipStream_t st, const MatSet& ms, size_t k, Quan
     if ((rows + 15) / 16 * gemm_col_tiles(ms, 16) <= kDirectTiles16)
         return launch_gemm_direct(st, SEM_FMA_CHAIN, ms, k, x, rows, dbg);
     if ((rows + 63) / 64 * gemm_col_tiles(ms, 64) <= kChainTiles64)
-        launch_q8<SEM_FMA_CHAIN, 64, 64, 1, 4, 4, 3, 2, 1>(st, ms, x, rows, k, dbg);
+        launch_q8<SEM_FMA_CHAIN, 64, 64, 1, 4, 4, 3, 2, 2>(st, ms, x, rows, k, dbg);
     else
         launch_q8<SEM_FMA_CHAIN, 128, 128, 2, 4, 4, 2, 1, 1>(st, ms, x, rows, k, dbg);
     return hipGetLastError();
@@ -803,7 +803,7 @@ hipError_t launch_qkv_rope(hipStream_t st, const DevMatrix& q, const DevMatrix& 
     if (q.storage == KR_STORAGE_Q8_0X4) {
         if (qkv_rope_direct(q, k, rows)) return launch_direct_rope(st, SEM_FMA_CHAIN, ms, q.k, x, rows, ro);
         if ((rows + 63) / 64 * ((q.n + 2 * k.n) / 64) <= kChainTiles64)
-            launch_q8_rope<SEM_FMA_CHAIN, 64, 64, 1, 4, 4, 3, 2, 1>(st, ms, x, rows, q.k, ro);
+            launch_q8_rope<SEM_FMA_CHAIN, 64, 64, 1, 4, 4, 3, 2, 2>(st, ms, x, rows, q.k, ro);
         else
             launch_q8_rope<SEM_FMA_CHAIN, 128, 128, 2, 4, 4, 2, 1, 1>(st, ms, x, rows, q.k, ro);
         return hipGetLastError();
@@ -850,7 +850,7 @@ hipError_t launch_gate_up_silu(hipStream_t st, const DevMatrix& gate, const DevM
     if (gate.storage == KR_STORAGE_Q8_0X4) {
         if (direct <= kDirectSwiMax) return launch_direct_swi(st, SEM_FMA_CHAIN, ms, gate.k, x, rows, so);
         if ((rows + 63) / 64 * blocks <= kChainTiles64)
-            launch_q8_swi<SEM_FMA_CHAIN, 64, 64, 1, 4, 4, 3, 2, 1>(st, ms, x, rows, gate.k, so);
+            launch_q8_swi<SEM_FMA_CHAIN, 64, 64, 1, 4, 4, 3, 2, 2>(st, ms, x, rows, gate.k, so);
         else
             launch_q8_swi<SEM_FMA_CHAIN, 128, 128, 2, 4, 4, 2, 1, 1>(st, ms, x, rows, gate.k, so);
         return hipGetLastError();

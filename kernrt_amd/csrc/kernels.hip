@@ -1998,7 +1998,7 @@ __global__ __launch_bounds__(1024) void k_attn_softmax_v(const float* __restrict
     const DevWindow w = win[row];
     sc_in += (size_t)row * n_heads * ss;
     mxp += (size_t)row * n_heads * ms;
-    att += (size_t)row * n_heads * seq_len;
+    if (att) att += (size_t)row * n_heads * seq_len;
     out += (size_t)row * n_heads * HS;
     const uint32_t n_shared = w.shared_end - w.shared_start;
     const uint32_t count = n_shared + w.slot - w.att_start + 1;  // <= scs
@@ -2072,7 +2072,7 @@ __global__ __launch_bounds__(1024) void k_attn_softmax_v(const float* __restrict
     // window): waves 8-15 store the pass's V slice transposed (the first pass
     // while the softmax sums run), all waves form the pass's probabilities
     // and products, and the chain lanes continue their sums over them
-    constexpr uint32_t NL = G * DW;
+    constexpr uint32_t NL = G * DW, NLW = (NL + 63) & ~63u;  // the chain lanes, whole waves of them
     float* prod = vt + DW * vst;
     float acc = 0.0f;  // lane tid < NL: the running V sum of (head tid / DW, dim tid % DW)
     float sj[G];
@@ -2124,10 +2124,10 @@ __global__ __launch_bounds__(1024) void k_attn_softmax_v(const float* __restrict
         const bool last = p0 + pw >= count;
         if (tid < NL) {
             acc = chain_sum(prod + tid * vst, n32, acc);
-        } else if (last && sidx == 0 && tid >= 64) {
+        } else if (att && last && sidx == 0 && tid >= NLW) {
             // the probabilities to `att` while the chains run (global stores
             // issued earlier would hold up every later wait on the memory counter)
-            for (uint32_t t = tid - 64; t < G * count; t += T - 64) {
+            for (uint32_t t = tid - NLW; t < G * count; t += T - NLW) {
                 const uint32_t j = t / count, i = t - j * count;
                 att[(size_t)(hk * G + j) * seq_len + i] = ps[j * scs + i];
             }
@@ -2144,11 +2144,25 @@ static constexpr size_t kAttnSplitDW = 4;
 // positions per pass of k_attn_softmax_v's V slice and product table: the
 // whole window in one pass where the LDS holds it, else the fewest passes
 // (of whole 64-position chunks) that fit beside the G score rows; 0: none do
-static size_t attn_split_pass(size_t scs, size_t G) {
+static size_t attn_split_pass(size_t scs, size_t G, size_t dw = kAttnSplitDW) {
     for (size_t np = 1; np <= 16; np++) {
         const size_t pw = ((scs + np - 1) / np + 63) & ~(size_t)63;
-        if (attn_split_lds(scs, G, kAttnSplitDW, pw) <= kAttnSplitLds) return pw;
+        if (attn_split_lds(scs, G, dw, pw) <= kAttnSplitLds) return pw;
     }
+    return 0;
+}
+
+// Output dims per k_attn_softmax_v workgroup for `blocks` (row, KV head) pairs,
+// 0: k_attn_softmax_v_rows, a workgroup per pair. Slices spread a pair over
+// more CUs but each repeats its softmax, so they pay while the whole grid fits
+// one workgroup per CU; 16 dims where 4 would not. us, slices of 4 / 16 /
+// pair: 15/5 heads of 64, 1 x 520 11.1 / 14.8 / 22.2, 3 x 300 10.2 / 12.4 /
+// 16.0, 6 x 400 16.7 / 14.4 / 19.5, 12 x 300 24.8 / 15.5 / 16.8, 16 x 250 28 /
+// 21.7 / 15.2; 16/8 heads of 128, 1 x 3000 35 / 44 / 85, 4 x 1000 46 / 27 / 36.
+static size_t attn_slice_dims(size_t blocks, size_t max_count, size_t G, size_t hs) {
+    const size_t scs = (max_count + 3) & ~(size_t)3;
+    if (blocks * (hs / 4) <= 256 && attn_split_pass(scs, G, 4) > 0) return 4;
+    if (blocks * (hs / 16) <= 256 && max_count <= 64 * 64 && attn_split_pass(scs, G, 16) > 0) return 16;
     return 0;
 }
 
@@ -2166,6 +2180,12 @@ bool attention_split_rows_ok(size_t max_count, size_t kv_mul, size_t hs) {
     if (hs != 32 && hs != 64 && hs != 128) return false;
     const size_t scs = (max_count + 3) & ~(size_t)3;
     return max_count >= 1 && max_count <= 16384 && (kv_mul * scs + 64 * hs) * sizeof(float) <= kAttnSplitLds;
+}
+
+// The window length that the many-row form's scratch is laid out for: in steps,
+// so that windows that grow by a token a step seldom move it.
+size_t attention_split_cap(size_t max_count, size_t seq_len) {
+    return std::min((max_count + 511) & ~(size_t)511, seq_len);
 }
 
 // scores [n_heads][round4(seq_len)] | chunk maxima [n_heads][attn_split_ms(seq_len)]
@@ -2186,8 +2206,10 @@ hipError_t launch_attention_split(hipStream_t st, const float* q, const float* k
     const uint32_t ss = (uint32_t)((seq_len + 3) & ~(size_t)3);  // scratch row stride
     const uint32_t ms = (uint32_t)attn_split_ms(seq_len);
     float* mxp = scratch + n_heads * ss;
-    const size_t pw = attn_split_pass(scs, kv_mul), lds = attn_split_lds(scs, kv_mul, kAttnSplitDW, pw);
-    const dim3 g1((unsigned)n_kv, (unsigned)nchunks), g2((unsigned)(n_kv * (hs / kAttnSplitDW)));
+    // 16 dims a workgroup where 4 would not leave each its CU (32 KV heads of 64, 200 positions: 9.5 against 11.9 us)
+    const size_t dw = attn_slice_dims(n_kv, max_count, kv_mul, hs) == 16 ? 16 : kAttnSplitDW;
+    const size_t pw = attn_split_pass(scs, kv_mul, dw), lds = attn_split_lds(scs, kv_mul, dw, pw);
+    const dim3 g1((unsigned)n_kv, (unsigned)nchunks), g2((unsigned)(n_kv * (hs / dw)));
 #define KR_SPLIT(G, H)                                                                                              \
     do {                                                                                                            \
         if (qnw || knw)                                                                                             \
@@ -2198,7 +2220,10 @@ hipError_t launch_attention_split(hipStream_t st, const float* q, const float* k
             hipLaunchKernelGGL((k_attn_scores<G, H, true>), g1, dim3(64), 0, st, q, k, v, kc, vc, loff, window, pos, \
                                table, interleaved, (uint32_t)kv_dim, scale, sc, ss, mxp, ms, (uint32_t)(n_heads * hs), \
                                nullptr, nullptr, 0.0f);                                                             \
-        if (max_count > 64 * 64)                                                                                    \
+        if (dw == 16)                                                                                               \
+            hipLaunchKernelGGL((k_attn_softmax_v<G, H, 16>), g2, dim3(1024), lds, st, sc, ss, mxp, ms, vc, loff,     \
+                               window, (uint32_t)kv_dim, (uint32_t)seq_len, (uint32_t)scs, att, out, (uint32_t)pw); \
+        else if (max_count > 64 * 64)                                                                               \
             hipLaunchKernelGGL((k_attn_softmax_v<G, H, kAttnSplitDW, true>), g2, dim3(1024), lds, st, sc, ss, mxp,  \
                                ms, vc, loff, window, (uint32_t)kv_dim, (uint32_t)seq_len, (uint32_t)scs, att, out,  \
                                (uint32_t)pw);                                                                       \
@@ -2481,7 +2506,7 @@ __global__ __launch_bounds__(64 * NWAVES) void k_attn_rows(const float* __restri
                                                    uint32_t n_heads, uint32_t kv_mul, uint32_t kv_dim,
                                                    uint32_t seq_len, float scale, uint32_t scs,
                                                    int8_t* __restrict__ qo, float* __restrict__ so,
-                                                   uint16_t* __restrict__ ho) {
+                                                   uint16_t* __restrict__ ho, const uint32_t* __restrict__ blocks) {
     using Sh = AttnRowsShape<HS, NWAVES>;
     constexpr uint32_t NW = Sh::NW, NT = Sh::NT, LPR = Sh::LPR, RPW = Sh::RPW, T = Sh::T, F = HS / 4;
     constexpr uint32_t NH = Sh::NH, FK = Sh::FK, KSK = Sh::KSK, TV = Sh::TV, KSV = Sh::KSV;
@@ -2495,8 +2520,9 @@ __global__ __launch_bounds__(64 * NWAVES) void k_attn_rows(const float* __restri
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // the last row blocks first: a causal prefill's windows grow with the
     // row, so the longest blocks start first and the short ones fill in behind
-    const uint32_t r0 = (gridDim.y - 1 - blockIdx.y) * R;
-    const uint32_t nr = min(R, n_rows - r0);
+    const uint32_t bi = gridDim.y - 1 - blockIdx.y;
+    const uint32_t r0 = blocks ? blocks[bi] : bi * R;
+    const uint32_t nr = blocks ? blocks[bi + 1] - r0 : min(R, n_rows - r0);
     // query heads h0 .. h0 + G - 1 of KV head h0 / kv_mul (G divides kv_mul)
     const uint32_t width = n_heads * HS, h0 = blockIdx.x * G, kvo = (h0 / kv_mul) * HS;
     const DevWindow w0 = windows[r0];
@@ -2996,11 +3022,16 @@ hipError_t launch_attention_split_rows(hipStream_t st, const float* q, float* ou
         return hipErrorInvalidValue;
     const size_t n_kv = n_heads / kv_mul, nchunks = (max_count + 63) / 64, loff = layer * seq_len * kv_dim;
     const size_t scs = (max_count + 3) & ~(size_t)3;
-    const uint32_t ss = (uint32_t)((seq_len + 3) & ~(size_t)3), ms = (uint32_t)attn_split_ms(seq_len);
+    const size_t cap = attention_split_cap(max_count, seq_len);  // the scratch's row stride
+    const uint32_t ss = (uint32_t)((cap + 3) & ~(size_t)3), ms = (uint32_t)attn_split_ms(cap);
     float* sc = scratch;
     float* mxp = scratch + n_rows * n_heads * ss;
     const size_t lds = (kv_mul * scs + 64 * hs) * sizeof(float);
     const dim3 g1((unsigned)n_kv, (unsigned)nchunks, (unsigned)n_rows), g2((unsigned)n_kv, (unsigned)n_rows);
+    const size_t dw = attn_slice_dims(n_rows * n_kv, max_count, kv_mul, hs), dws = dw ? dw : kAttnSplitDW;
+    const size_t pw = attn_split_pass(scs, kv_mul, dws), lds3 = attn_split_lds(scs, kv_mul, dws, pw);
+    const dim3 g3((unsigned)(n_kv * (hs / dws)), (unsigned)n_rows);
+    if (!keep_att) att = nullptr;
     float* kcw = const_cast<float*>(kc);  // written only by the RoPE form
     float* vcw = const_cast<float*>(vc);
 #define KR_SPLIT_ROWS(G, H)                                                                                          \
@@ -3008,9 +3039,20 @@ hipError_t launch_attention_split_rows(hipStream_t st, const float* q, float* ou
         hipLaunchKernelGGL((k_attn_scores<G, H, false>), g1, dim3(64), 0, st, q, nullptr, nullptr, kcw, vcw, loff,   \
                            windows, nullptr, nullptr, 0, (uint32_t)kv_dim, scale, sc, ss, mxp, ms,                   \
                            (uint32_t)(n_heads * hs), nullptr, nullptr, 0.0f);                                        \
-        hipLaunchKernelGGL((k_attn_softmax_v_rows<G, H>), g2, dim3(G * H < 64 ? 64 : G * H), lds, st, sc, ss, mxp, ms, \
-                           vc, loff, windows, (uint32_t)kv_dim, (uint32_t)seq_len, (uint32_t)scs, (uint32_t)n_heads,  \
-                           keep_att ? att : nullptr, out, qo, so, ho);                                                \
+        if (dw == 4 && max_count > 64 * 64)                                                                          \
+            hipLaunchKernelGGL((k_attn_softmax_v<G, H, 4, true>), g3, dim3(1024), lds3, st, sc, ss, mxp, ms, vc,     \
+                               loff, windows, (uint32_t)kv_dim, (uint32_t)seq_len, (uint32_t)scs, att, out,          \
+                               (uint32_t)pw);                                                                        \
+        else if (dw == 4)                                                                                            \
+            hipLaunchKernelGGL((k_attn_softmax_v<G, H, 4>), g3, dim3(1024), lds3, st, sc, ss, mxp, ms, vc, loff,     \
+                               windows, (uint32_t)kv_dim, (uint32_t)seq_len, (uint32_t)scs, att, out, (uint32_t)pw); \
+        else if (dw == 16)                                                                                           \
+            hipLaunchKernelGGL((k_attn_softmax_v<G, H, 16>), g3, dim3(1024), lds3, st, sc, ss, mxp, ms, vc, loff,    \
+                               windows, (uint32_t)kv_dim, (uint32_t)seq_len, (uint32_t)scs, att, out, (uint32_t)pw); \
+        else                                                                                                         \
+            hipLaunchKernelGGL((k_attn_softmax_v_rows<G, H>), g2, dim3(G * H < 64 ? 64 : G * H), lds, st, sc, ss, mxp, \
+                               ms, vc, loff, windows, (uint32_t)kv_dim, (uint32_t)seq_len, (uint32_t)scs,             \
+                               (uint32_t)n_heads, att, out, qo, so, ho);                                              \
     } while (0)
 #define KR_SPLIT_ROWS_H(G)       \
     if (hs == 32)                \
@@ -3028,21 +3070,63 @@ hipError_t launch_attention_split_rows(hipStream_t st, const float* q, float* ou
     }
 #undef KR_SPLIT_ROWS_H
 #undef KR_SPLIT_ROWS
+    if (dw && qo) return launch_quantize(st, out, n_rows, n_heads * hs, n_heads * hs, qo, so, ho);
     return hipGetLastError();
 }
 
-// Whether a block of rows can run k_attn_rows: its windows share att_start
-// and the shared range (prefill), checked per block of the kernel's R rows.
-bool attention_rows_uniform(const DevWindow* w, size_t n_rows, size_t max_count, size_t kv_mul, size_t hs) {
-    const size_t G = attn_rows_group(kv_mul), nw = attn_rows_waves(G, hs, max_count);
-    if (n_rows < 2 || nw == 0) return false;
-    const size_t R = (nw * (128 / hs)) / G;
+// Row blocks of at most R rows whose windows share att_start and the shared
+// range: the first row of each, then n_rows; empty where every R rows do.
+static std::vector<uint32_t> attn_blocks(const DevWindow* w, size_t n_rows, size_t R) {
+    std::vector<uint32_t> b;
+    bool regular = true;
     for (size_t r = 0; r < n_rows; r++) {
-        const DevWindow& a = w[r - r % R];
-        if (a.att_start != w[r].att_start || a.shared_start != w[r].shared_start || a.shared_end != w[r].shared_end)
-            return false;
+        const DevWindow& a = w[b.empty() ? 0 : b.back()];
+        if (b.empty() || r - b.back() == R || a.att_start != w[r].att_start || a.shared_start != w[r].shared_start ||
+            a.shared_end != w[r].shared_end) {
+            regular = regular && r % R == 0;
+            b.push_back((uint32_t)r);
+        }
     }
-    return true;
+    if (regular && b.size() == (n_rows + R - 1) / R) return {};
+    b.push_back((uint32_t)n_rows);
+    return b;
+}
+
+// Which launches take `n_rows` rows with the given windows. Rows whose blocks
+// share a window layout (a prefill, also of several sequences, whose blocks the
+// table keeps apart) can run by blocks: on the matrix core (attn_mx.hip) for
+// long windows, else k_attn_rows. Both are as long as their longest block
+// however few there are, so up to some number of (row, KV head) pairs the
+// per-row launches are shorter. us, blocks / per row: 15/5 heads of 64, 9 rows
+// at 512 36 / 18, 128 rows at 512 42.9 / 41.4, 32 rows at 2000 224 / 74, 200
+// rows at 900 133 / 94; 32/32 heads of 64, 16 rows at 200 19.0 / 16.9, 64 rows
+// 22 / 36; 64 rows at 900 120 / 136; 16/8 heads of 128, 32 rows at 0 18.9 / 9.3,
+// 200 rows at 100 53 / 42, 250 rows at 0 44 / 43, 128 rows at 1500 214 / 149.
+// Sequences of their own lengths, blocks by the table: 24 of 700 rows in all,
+// 15/5 heads 19.9 / 30.8, 16/8 heads of 128 108 / 62; 8 of 1500 rows 89 / 247.
+AttnPlan attention_plan(const DevWindow* w, size_t n_rows, size_t max_count, size_t n_heads, size_t kv_mul,
+                        size_t hs) {
+    AttnPlan p;
+    const size_t pairs = n_rows * (n_heads / kv_mul);
+    const bool split = attention_split_rows_ok(max_count, kv_mul, hs);
+    if (n_rows < 2) {  // k_attention_fast up to 256 positions of small heads (9 against 9.5 us)
+        if (split && (max_count >= 256 || hs == 128)) p.kind = ATTN_SPLIT;
+        return p;
+    }
+    auto blocked = [&](size_t R) {  // blocks at least half full, or the regular ones
+        p.blocks = attn_blocks(w, n_rows, R);
+        return p.blocks.empty() || (R > 1 && (p.blocks.size() - 1) * R <= 2 * n_rows);
+    };
+    const size_t nw = attn_rows_waves(attn_rows_group(kv_mul), hs, max_count);
+    if (attention_mx_rows(max_count, kv_mul, hs) && blocked(attention_mx_rows(max_count, kv_mul, hs))) {
+        p.kind = split && pairs <= (hs == 128 ? 1792 : 1280) ? ATTN_SPLIT : ATTN_MX;
+    } else if (nw && blocked(nw * (128 / hs) / attn_rows_group(kv_mul))) {
+        p.kind = split && (hs == 128 || (max_count > 64 && pairs <= 512)) ? ATTN_SPLIT : ATTN_ROWS;
+    } else {
+        p.kind = split ? ATTN_SPLIT : ATTN_GENERAL;
+    }
+    if (p.kind == ATTN_SPLIT || p.kind == ATTN_GENERAL) p.blocks.clear();
+    return p;
 }
 
 // LDS budget of the latency-first attention and its shape for one call:
@@ -3084,27 +3168,29 @@ hipError_t launch_attention(hipStream_t st, const float* q, float* out, float* a
                             const float* vc, size_t layer, const DevWindow* windows, size_t n_rows,
                             size_t max_count, size_t n_heads, size_t kv_mul, size_t hs, size_t kv_dim,
                             size_t seq_len, float scale, int8_t* qo, float* so, uint16_t* ho,
-                            const DevWindow* host_windows, float* mx_scratch, bool keep_att) {
+                            const AttnPlan& plan, const uint32_t* blocks, float* mx_scratch, bool keep_att) {
     if (n_rows == 0) return hipSuccess;
     if (hs == 0 || hs > 256 || hs % 4 != 0 || kv_mul == 0 || n_heads % kv_mul != 0) return hipErrorInvalidValue;
     if (qo && hs % 32 != 0) return hipErrorInvalidValue;
     if (max_count > seq_len) max_count = seq_len;
-    if (host_windows && mx_scratch && attention_mx_ok(host_windows, n_rows, max_count, kv_mul, hs)) {
+    if (plan.blocks.empty()) blocks = nullptr;
+    const size_t n_blocks = plan.blocks.empty() ? 0 : plan.blocks.size() - 1;
+    if (plan.kind == ATTN_MX && mx_scratch) {
         // blocks of 32 (row, head) pairs on the matrix core (attn_mx.hip)
         return launch_attention_mx(st, q, out, att, kc, vc, layer, windows, n_rows, max_count, n_heads, kv_mul, hs,
-                                   kv_dim, seq_len, scale, qo, so, ho, mx_scratch, keep_att);
+                                   kv_dim, seq_len, scale, qo, so, ho, mx_scratch, keep_att, blocks, n_blocks);
     }
-    if (host_windows && attention_rows_uniform(host_windows, n_rows, max_count, kv_mul, hs)) {
+    if (plan.kind == ATTN_ROWS) {
         // many rows whose blocks share a window layout: k_attn_rows
         const size_t G = attn_rows_group(kv_mul), nw = attn_rows_waves(G, hs, max_count);
         const size_t R = (nw * (128 / hs)) / G;  // rows per block: AttnRowsShape
         const size_t lds = attn_rows_lds(G, hs, max_count, nw);
         const uint32_t scs = (uint32_t)((max_count + 3) & ~(size_t)3);
-        const dim3 grid((unsigned)(n_heads / G), (unsigned)((n_rows + R - 1) / R));
+        const dim3 grid((unsigned)(n_heads / G), (unsigned)(blocks ? n_blocks : (n_rows + R - 1) / R));
 #define KR_ATTN_ROWS(g, h, w)                                                                                 \
     hipLaunchKernelGGL((k_attn_rows<g, h, w>), grid, dim3(64 * w), lds, st, q, out, keep_att ? att : nullptr, kc,   \
                        vc, layer * seq_len * kv_dim, windows, (uint32_t)n_rows, (uint32_t)n_heads,              \
-                       (uint32_t)kv_mul, (uint32_t)kv_dim, (uint32_t)seq_len, scale, scs, qo, so, ho)
+                       (uint32_t)kv_mul, (uint32_t)kv_dim, (uint32_t)seq_len, scale, scs, qo, so, ho, blocks)
 #define KR_ATTN_ROWS_W(g, h)         \
     if (nw == 8)                     \
         KR_ATTN_ROWS(g, h, 8);       \

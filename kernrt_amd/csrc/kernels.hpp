@@ -7,6 +7,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <vector>
+
 namespace kr {
 
 // Output-order semantics of a quantized projection (the reference's f32
@@ -110,22 +112,32 @@ hipError_t launch_kv_write(hipStream_t st, float* kc, float* vc, size_t layer, s
                            size_t kv_dim, const uint32_t* slots, const float* k, const float* v,
                            size_t rows);
 struct DevWindow { uint32_t att_start, slot, shared_start, shared_end; };
+// Which launches an attention call takes (attention_plan). `blocks`: the first
+// row of each block of rows that share a window layout, then the row count
+// (empty: the blocks are regular); launch_attention takes its device copy.
+enum AttnKind { ATTN_GENERAL, ATTN_ROWS, ATTN_MX, ATTN_SPLIT };
+struct AttnPlan {
+    AttnKind kind = ATTN_GENERAL;
+    std::vector<uint32_t> blocks;
+};
+AttnPlan attention_plan(const DevWindow* host_windows, size_t n_rows, size_t max_count, size_t n_heads, size_t kv_mul,
+                        size_t hs);
 hipError_t launch_attention(hipStream_t st, const float* q, float* out, float* att, const float* kc,
                             const float* vc, size_t layer, const DevWindow* windows, size_t n_rows,
                             size_t max_count, size_t n_heads, size_t kv_mul, size_t head_size,
                             size_t kv_dim, size_t seq_len, float scale, int8_t* qo = nullptr,
-                            float* so = nullptr, uint16_t* ho = nullptr, const DevWindow* host_windows = nullptr,
-                            float* mx_scratch = nullptr, bool keep_att = true);
-// Prefill attention on the matrix core (attn_mx.hip): whether a launch can
-// take it (head size 64 or 128, a longest window of 1024 to 4096 positions,
-// every block of 32 / G rows sharing one window layout), and the launch.
-bool attention_mx_ok(const DevWindow* w, size_t n_rows, size_t max_count, size_t kv_mul, size_t hs);
+                            float* so = nullptr, uint16_t* ho = nullptr, const AttnPlan& plan = {},
+                            const uint32_t* blocks = nullptr, float* mx_scratch = nullptr, bool keep_att = true);
+// Prefill attention on the matrix core (attn_mx.hip): the rows of its blocks,
+// which share one window layout (0: it does not take this head size or longest
+// window), and the launch.
+size_t attention_mx_rows(size_t max_count, size_t kv_mul, size_t hs);
 // `scratch` holds 2 n_rows n_heads floats (each pair's max and sum).
 hipError_t launch_attention_mx(hipStream_t st, const float* q, float* out, float* att, const float* kc,
                                const float* vc, size_t layer, const DevWindow* windows, size_t n_rows,
                                size_t max_count, size_t n_heads, size_t kv_mul, size_t hs, size_t kv_dim,
                                size_t seq_len, float scale, int8_t* qo, float* so, uint16_t* ho, float* scratch,
-                               bool keep_att = true);
+                               bool keep_att, const uint32_t* blocks, size_t n_blocks);
 // Decode attention of one row in two launches (scores by 64-row chunks with
 // RoPE and the kv_write of k/v folded in, and the per-head q / k RMSNorm
 // where qnw / knw are given, then softmax + V by head slices of 4 dims);
@@ -135,6 +147,7 @@ bool attention_split_ok(size_t max_count, size_t kv_mul, size_t hs);
 // launch_attention_split_rows's geometry check (k_attn_softmax_v_rows).
 bool attention_split_rows_ok(size_t max_count, size_t kv_mul, size_t hs);
 size_t attention_split_scratch(size_t n_heads, size_t seq_len);
+size_t attention_split_cap(size_t max_count, size_t seq_len);
 hipError_t launch_attention_split(hipStream_t st, const float* q, const float* k, const float* v, float* out,
                                   float* att, float* kc, float* vc, size_t layer, const DevWindow* window,
                                   const uint32_t* pos, const float2* table, int interleaved, size_t max_count,
@@ -143,7 +156,8 @@ hipError_t launch_attention_split(hipStream_t st, const float* q, const float* k
                                   const float* knw = nullptr, float eps = 0.0f);
 // The same two launches for many rows with windows of their own (batched
 // decode): q rows already rotated, keys already in the cache; `scratch`
-// holds n_rows * attention_split_scratch(n_heads, seq_len) floats. keep_att
+// holds n_rows * attention_split_scratch(n_heads, attention_split_cap(max_count,
+// seq_len)) floats. keep_att
 // false leaves `att` unwritten; qo/so/ho (head size a multiple of 32) take
 // the output rows' Q8 blocks as well.
 hipError_t launch_attention_split_rows(hipStream_t st, const float* q, float* out, float* att, const float* kc,
@@ -151,10 +165,6 @@ hipError_t launch_attention_split_rows(hipStream_t st, const float* q, float* ou
                                        size_t max_count, size_t n_heads, size_t kv_mul, size_t hs, size_t kv_dim,
                                        size_t seq_len, float scale, float* scratch, bool keep_att = true,
                                        int8_t* qo = nullptr, float* so = nullptr, uint16_t* ho = nullptr);
-// whether the rows' windows let launch_attention use its block-of-rows
-// (prefill) kernel: each block of rows shares att_start and the shared range
-bool attention_rows_uniform(const DevWindow* host_windows, size_t n_rows, size_t max_count, size_t kv_mul,
-                            size_t hs);
 hipError_t launch_add(hipStream_t st, float* dst, const float* src, size_t n);
 hipError_t launch_add_planes(hipStream_t st, float* dst, const float* planes, size_t n);
 hipError_t launch_mul(hipStream_t st, float* out, const float* a, const float* b, size_t n,

@@ -1,0 +1,52 @@
+"""The choice of attention launches (attention_plan) on both sides of its lines:
+every window layout gives the oracle's outputs and probabilities bit for bit,
+whichever launches take it."""
+
+import pytest
+
+from test_gpu_ops import _attention_case
+
+pytestmark = pytest.mark.gpu
+
+
+def causal(n, start=0, base=0, shared=0):
+    return [(base, base + start + i, 0, shared) for i in range(n)]
+
+
+def ragged(lens, shared=0):
+    out, base = [], shared
+    for n in lens:
+        out += causal(n, 0, base, shared)
+        base += n
+    return out
+
+
+# one row: below and at the split's first window, 4- and 16-dim slices (n_kv hs
+# / 4 workgroups up to and past 256), passes of the V slice
+@pytest.mark.parametrize("n_heads,n_kv,hs,count", [
+    (15, 5, 64, 255), (15, 5, 64, 256), (32, 32, 64, 700), (16, 8, 128, 3), (32, 16, 128, 2900), (4, 2, 32, 300),
+])
+def test_one_row(n_heads, n_kv, hs, count):
+    _attention_case(count + 5, n_heads, n_kv, hs, [(2, count + 1, 0, 0)], count)
+
+
+# few rows at long windows: slices of 4 and 16 dims, a workgroup per (row, KV
+# head), and blocks beyond the number of pairs that the per-row launches take
+@pytest.mark.parametrize("n_heads,n_kv,hs,n,start", [
+    (15, 5, 64, 3, 300), (15, 5, 64, 12, 290), (15, 5, 64, 13, 290), (6, 2, 64, 256, 70), (6, 2, 64, 257, 70),
+    (4, 4, 64, 30, 800), (16, 8, 128, 2, 150), (16, 8, 128, 30, 150), (16, 8, 128, 225, 3), (8, 8, 32, 65, 60),
+])
+def test_rows_of_one_sequence(n_heads, n_kv, hs, n, start):
+    _attention_case(start + n + 3, n_heads, n_kv, hs, causal(n, start), n + start)
+
+
+# sequences whose lengths leave blocks of every size: block tables for
+# k_attn_rows (heads of 64) and for the matrix core (820 and 225 rows), with and
+# without a shared prefix; too ragged for blocks; a row alone at the end
+@pytest.mark.parametrize("n_heads,n_kv,hs,lens,shared", [
+    (15, 5, 64, [1, 5, 6, 37, 64, 3, 2, 1], 0), (15, 5, 64, [70, 33, 48], 9), (4, 4, 64, [7, 50, 1, 9], 20),
+    (6, 2, 64, [1, 1, 2, 1, 1], 0), (16, 8, 128, [100, 30, 66, 1], 0), (16, 8, 128, [180, 17, 1, 15], 12), (16, 8, 128, [180, 17, 1, 30], 12),
+    (4, 2, 64, [790, 30, 1], 0), (8, 4, 32, [40, 3, 25], 7),
+])
+def test_rows_of_ragged_sequences(n_heads, n_kv, hs, lens, shared):
+    _attention_case(shared + sum(lens) + 2, n_heads, n_kv, hs, ragged(lens, shared), sum(lens) + shared)
