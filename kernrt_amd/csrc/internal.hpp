@@ -43,8 +43,10 @@ int greedy_step(kr_ctx* c, kr_buf logits, size_t len, uint32_t* step);
 // x += add (add may be KR_NO_BUF), out = rms_norm(x, w), quantize(out)
 int norm_quant(kr_ctx* c, kr_buf x, kr_buf add, int add_planes, kr_buf w, kr_buf out, size_t rows, size_t dim,
                float eps, bool chain_major = false);
-// dst += ((p0 + p1) + p2) + p3 over the four planes of a chain-split projection
-int add_planes(kr_ctx* c, kr_buf dst, kr_buf planes, size_t len);
+// norm_quant of the rows from[0..rows-1] of x (+= add, whose planes hold x_rows
+// rows) into rows 0..rows-1 of `out` and of the workspace
+int norm_quant_from(kr_ctx* c, kr_buf x, kr_buf add, int add_planes, size_t x_rows, kr_buf w, kr_buf out,
+                    const size_t* from, size_t rows, size_t dim, float eps);
 // projections of the quantized workspace rows; one launch when they share in_dim and storage
 int project_q(kr_ctx* c, size_t layer, const int* projs, const kr_buf* ys, int n, size_t rows);
 // out[oo + r os + i] = a[ao + r as + i] * b[bo + r bs + i], r < rows, i < n, one launch
@@ -53,8 +55,8 @@ int mul_rows(kr_ctx* c, kr_buf out, size_t oo, size_t os, kr_buf a, size_t ao, s
              size_t bs, size_t rows, size_t n);
 // gate = silu(gate) * up, quantized
 int silu_quant(kr_ctx* c, kr_buf gate, kr_buf up, size_t rows, size_t width);
-// prefill FFN after the norm's quantization: gate/up + SiLU * up + Q8 in one
-// GEMM launch, then down into `out` (Q8_0 gate/up, rows >= 8)
+// batch FFN after the norm's quantization: gate/up + SiLU * up + Q8 in one
+// GEMM launch, then down into `out`
 bool ffn_swiglu_ok(kr_ctx* c, size_t layer, size_t rows);
 // max_planes 4: the down projection may run chain-split and leave its four
 // partial-sum planes in `out` (room for 4 x rows x dim); *planes says which

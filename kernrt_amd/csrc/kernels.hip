@@ -755,6 +755,10 @@ struct GemvPro {
     const float* w;  // PRO_NORM: norm weight
     float* x_out;    // PRO_NORM: x + add, written by workgroup 0 (may be null)
     float eps;
+    // PRO_QUANT: the quantized row, written by workgroup 0 (q null: not written)
+    int8_t* q = nullptr;
+    float* s = nullptr;
+    uint16_t* h = nullptr;
 };
 static constexpr int PRO_NORM = 1, PRO_QUANT = 3;
 
@@ -834,6 +838,10 @@ __device__ __forceinline__ void gemv_produce(const GemvPro& pro, uint32_t K, flo
             // the block scale as the epilogue uses it: f16-rounded and widened
             // (quant.rs:276-288) for the FMA-chain format, else the f32 scale
             if ((f & 7) == 0) xsb[f / 8] = f2u(XF16 ? f16w(f16_bits(d)) : d);
+            if (PRO == PRO_QUANT && blockIdx.x == 0 && pro.q) {
+                ((char4*)pro.q)[f] = qq;
+                if ((f & 7) == 0) pro.s[f / 8] = d, pro.h[f / 8] = f16_bits(d);
+            }
         }
     }
     __syncthreads();
@@ -961,7 +969,7 @@ static hipError_t gemv_pro_go(hipStream_t st, MatSet ms, size_t k, const GemvPro
 
 hipError_t launch_project_pro(hipStream_t st, int sem, const DevMatrix* const* w, float* const* y, int count,
                               int pro_kind, const float* a, const float* b, const float* norm_w, float* x_out,
-                              float eps) {
+                              float eps, int8_t* q, float* s, uint16_t* h) {
     if (count < 1 || count > 3 || (pro_kind != PRO_NORM && pro_kind != PRO_QUANT)) return hipErrorInvalidValue;
     const size_t k = w[0]->k;
     if (k % 32 != 0 || k > 8192) return hipErrorInvalidValue;
@@ -975,7 +983,7 @@ hipError_t launch_project_pro(hipStream_t st, int sem, const DevMatrix* const* w
         ms.n[i] = (uint32_t)w[i]->n;
         ms.ld[i] = (uint32_t)w[i]->n;
     }
-    GemvPro pro{a, b, norm_w, x_out, eps};
+    GemvPro pro{a, b, norm_w, x_out, eps, q, s, h};
 #define KR_PRO_SEM(P)                                                                          \
     switch (sem) {                                                                             \
         case SEM_FMA_CHAIN: return gemv_pro_go<SEM_FMA_CHAIN, P>(st, ms, k, pro);              \
@@ -3292,12 +3300,13 @@ __global__ __launch_bounds__(256) void k_add_rms_quant(float* __restrict__ x, co
                                                        const float* __restrict__ w, float* __restrict__ out,
                                                        uint32_t dim, float eps, int8_t* __restrict__ q,
                                                        float* __restrict__ s, uint16_t* __restrict__ h,
-                                                       size_t pstride, uint32_t cm) {
+                                                       size_t pstride, uint32_t cm,
+                                                       const uint32_t* __restrict__ from) {
     extern __shared__ __align__(16) float sq[];  // [dim]
     __shared__ float s_scale;
     const uint32_t tid = threadIdx.x, n4 = dim / 4;
-    const size_t row = blockIdx.x;
-    float4* xr = (float4*)(x + row * dim);
+    const size_t row = blockIdx.x, src = from ? from[row] : row;
+    float4* xr = (float4*)(x + src * dim);
     float4 v[VPT], wv[VPT];
 #pragma unroll
     for (int u = 0; u < VPT; u++) {
@@ -3306,11 +3315,11 @@ __global__ __launch_bounds__(256) void k_add_rms_quant(float* __restrict__ x, co
             v[u] = xr[f];
             wv[u] = ((const float4*)w)[f];
             if (ADD) {
-                float4 a = ((const float4*)(add + row * dim))[f];
+                float4 a = ((const float4*)(add + src * dim))[f];
                 if (pstride) {
-                    const float4 a1 = ((const float4*)(add + pstride + row * dim))[f];
-                    const float4 a2 = ((const float4*)(add + 2 * pstride + row * dim))[f];
-                    const float4 a3 = ((const float4*)(add + 3 * pstride + row * dim))[f];
+                    const float4 a1 = ((const float4*)(add + pstride + src * dim))[f];
+                    const float4 a2 = ((const float4*)(add + 2 * pstride + src * dim))[f];
+                    const float4 a3 = ((const float4*)(add + 3 * pstride + src * dim))[f];
                     a = make_float4(((a.x + a1.x) + a2.x) + a3.x, ((a.y + a1.y) + a2.y) + a3.y,
                                     ((a.z + a1.z) + a2.z) + a3.z, ((a.w + a1.w) + a2.w) + a3.w);
                 }
@@ -3322,7 +3331,7 @@ __global__ __launch_bounds__(256) void k_add_rms_quant(float* __restrict__ x, co
     for (int u = 0; u < VPT; u++) {
         const uint32_t f = tid + 256 * u;
         if (f < n4) {
-            if (ADD) xr[f] = v[u];
+            if (ADD && !from) xr[f] = v[u];
             ((float4*)sq)[f] = make_float4(v[u].x * v[u].x, v[u].y * v[u].y, v[u].z * v[u].z, v[u].w * v[u].w);
         }
     }
@@ -3369,17 +3378,17 @@ __global__ __launch_bounds__(256) void k_add_rms_quant(float* __restrict__ x, co
 
 hipError_t launch_add_rms_quant(hipStream_t st, float* x, const float* add, const float* w, float* out,
                                 size_t rows, size_t dim, float eps, int8_t* q, float* s, uint16_t* h, int add_planes,
-                                bool chain_major) {
+                                bool chain_major, const uint32_t* from, size_t x_rows) {
     if (rows == 0) return hipSuccess;
     if (dim % 32 != 0 || dim > 8192 || (add_planes != 1 && add_planes != 4) || (chain_major && dim % 128 != 0))
         return hipErrorInvalidValue;
-    const size_t pstride = add_planes == 4 ? rows * dim : 0;
+    const size_t pstride = add_planes == 4 ? (from ? x_rows : rows) * dim : 0;
     const uint32_t cm = chain_major ? 1u : 0u;
     const size_t lds = dim * sizeof(float);
     const size_t vpt = (dim / 4 + 255) / 256;
 #define KR_NORM_GO(A, V)                                                                                        \
     hipLaunchKernelGGL((k_add_rms_quant<A, V>), dim3((unsigned)rows), dim3(256), lds, st, x, add, w, out,      \
-                       (uint32_t)dim, eps, q, s, h, pstride, cm)
+                       (uint32_t)dim, eps, q, s, h, pstride, cm, from)
 #define KR_NORM_V(A)          \
     if (vpt <= 1)             \
         KR_NORM_GO(A, 1);     \
@@ -3604,18 +3613,6 @@ __global__ void k_add(float* __restrict__ d, const float* __restrict__ s, size_t
 hipError_t launch_add(hipStream_t st, float* d, const float* s, size_t n) {
     if (n == 0) return hipSuccess;
     hipLaunchKernelGGL(k_add, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, d, s, n);
-    return hipGetLastError();
-}
-
-// d += ((p0 + p1) + p2) + p3 over the four partial-sum planes of a
-// chain-split projection, n floats each (dot.rs:45, then the residual add)
-__global__ void k_add_planes(float* __restrict__ d, const float* __restrict__ p, size_t n) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) d[i] = d[i] + (((p[i] + p[n + i]) + p[2 * n + i]) + p[3 * n + i]);
-}
-hipError_t launch_add_planes(hipStream_t st, float* d, const float* p, size_t n) {
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_add_planes, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, d, p, n);
     return hipGetLastError();
 }
 

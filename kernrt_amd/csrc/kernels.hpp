@@ -46,10 +46,13 @@ hipError_t launch_project_set(hipStream_t st, int sem, const DevMatrix* const* w
 // Fused decode/prefill steps (same arithmetic as the separate ops):
 // x += add (when add != null), out = rms_norm(x) and its Q8 quantization.
 // add_planes 4: `add` holds a chain-split projection's four partial-sum planes;
-// chain_major: the Q8 blocks in chain-major order (for launch_gemm_q8_cs)
+// chain_major: the Q8 blocks in chain-major order (for launch_gemm_q8_cs);
+// from (device): output row i takes row from[i] of x and add, which hold x_rows rows
+// (x is then left as it is)
 hipError_t launch_add_rms_quant(hipStream_t st, float* x, const float* add, const float* w, float* out,
                                 size_t rows, size_t dim, float eps, int8_t* q, float* s, uint16_t* h,
-                                int add_planes = 1, bool chain_major = false);
+                                int add_planes = 1, bool chain_major = false, const uint32_t* from = nullptr,
+                                size_t x_rows = 0);
 // g = silu(g) * u and its Q8 quantization, rows of `width`
 hipError_t launch_silu_quant(hipStream_t st, float* g, const float* u, size_t rows, size_t width, int8_t* q,
                              float* s, uint16_t* h);
@@ -67,7 +70,8 @@ hipError_t launch_qk_norm_rope_kv(hipStream_t st, float* q, float* k, const floa
 // y[m*ldy + n] for m < rows. Uses the GEMV path (rows <= 4) or the MFMA GEMM.
 // One decode row (M = 1) of 1-3 projections with the producer of their input
 // fused in front: pro_kind 1 = x (+= add) -> rms_norm(w, eps) -> Q8 (the
-// updated x row goes to x_out when non-null), 3 = Q8 of the f32 row a.
+// updated x row goes to x_out when non-null), 3 = Q8 of the f32 row a (which
+// also goes to (q, s, h) when q is non-null).
 // One decode row of gate/up with the producer in front (x (+= add) ->
 // rms_norm(norm_w, eps) -> Q8, the updated x row to x_out when non-null) and
 // h = silu(gate) * up behind, quantized into (hq, hs, hh) for the down
@@ -94,7 +98,7 @@ hipError_t launch_gate_up_swiglu(hipStream_t st, int sem, const DevMatrix& gate,
                                  float* hs, uint16_t* hh, float* hf);
 hipError_t launch_project_pro(hipStream_t st, int sem, const DevMatrix* const* w, float* const* y, int count,
                               int pro_kind, const float* a, const float* b, const float* norm_w, float* x_out,
-                              float eps);
+                              float eps, int8_t* q = nullptr, float* s = nullptr, uint16_t* h = nullptr);
 hipError_t launch_project(hipStream_t st, int sem, const DevMatrix& w, QuantAct x, size_t rows,
                           float* y, size_t ldy, int32_t* dbg_block_dots);
 
@@ -166,7 +170,6 @@ hipError_t launch_attention_split_rows(hipStream_t st, const float* q, float* ou
                                        size_t seq_len, float scale, float* scratch, bool keep_att = true,
                                        int8_t* qo = nullptr, float* so = nullptr, uint16_t* ho = nullptr);
 hipError_t launch_add(hipStream_t st, float* dst, const float* src, size_t n);
-hipError_t launch_add_planes(hipStream_t st, float* dst, const float* planes, size_t n);
 hipError_t launch_mul(hipStream_t st, float* out, const float* a, const float* b, size_t n,
                       int sequential);
 // o[r os + i] = a[r as + i] * b[r bs + i] for r < rows, i < n (no overlap of o with a or b)

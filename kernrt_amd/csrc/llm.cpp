@@ -378,8 +378,15 @@ int prefill_conv(krl_model* m, size_t l, size_t n_tok, bool stepped) {
 
 // llama.rs:690-771, generalised with the LFM2 conv branch of lfm2.rs:559-632.
 // `stepped_conv`: the conv layers reproduce a token-by-token prefill
-// (prefill_conv).
-int prefill_rows(krl_model* m, const std::vector<Row>& rows, bool stepped_conv = false) {
+// (prefill_conv). With the fused kernels the last layer's down projection is
+// left to the final norm to add (`last`: p.o, as one plane or four); else
+// p.x is complete and last->add is KR_NO_BUF.
+struct LastAdd {
+    kr_buf add = KR_NO_BUF;
+    int planes = 1;
+    size_t rows = 0;
+};
+int prefill_rows(krl_model* m, const std::vector<Row>& rows, LastAdd* last, bool stepped_conv = false) {
     kr_ctx* b = m->b;
     Geometry g = geometry(m->c);
     size_t n_tok = rows.size();
@@ -400,8 +407,7 @@ int prefill_rows(krl_model* m, const std::vector<Row>& rows, bool stepped_conv =
         for (size_t r = 0; r < n_tok; r++) KRC(m, kr_embed(b, rows[r].token, p.x, r * g.dim));
     }
     if (m->fused) {
-        // prefill_rows with the fused kernels (see decode_step_fused); the
-        // last residual add is applied here because the final norm reads one row
+        // prefill_rows with the fused kernels (see decode_step_fused)
         // `pending` is the last projection into the residual stream, one plane
         // or a chain-split projection's four partial-sum planes
         kr_buf pending = KR_NO_BUF;
@@ -466,10 +472,9 @@ int prefill_rows(krl_model* m, const std::vector<Row>& rows, bool stepped_conv =
             }
             pending = p.o;
         }
-        if (planes == 4)
-            KRC(m, kri::add_planes(b, p.x, pending, n_tok * g.dim));
-        else
-            KRC(m, kr_add_in_place(b, p.x, pending, n_tok * g.dim));
+        last->add = pending;
+        last->planes = planes;
+        last->rows = n_tok;
         return KR_OK;
     }
     for (size_t l = 0; l < m->c.n_layers; l++) {
@@ -503,9 +508,30 @@ int prefill_rows(krl_model* m, const std::vector<Row>& rows, bool stepped_conv =
     return KR_OK;
 }
 
-// llama.rs:652-683
-int final_hiddens(krl_model* m, const std::vector<long>& rows, float* out) {
-    size_t dim = m->c.dim;
+// llama.rs:652-683: the final-normed hidden rows `rows` (zeros for < 0). With the
+// fused kernels one launch and one read for all of them.
+int final_hiddens(krl_model* m, const std::vector<long>& rows, const LastAdd& last, float* out) {
+    const size_t dim = m->c.dim;
+    if (last.add != KR_NO_BUF) {
+        std::vector<size_t> from;
+        for (long r : rows)
+            if (r >= 0) from.push_back((size_t)r);
+        KRC(m, kri::norm_quant_from(m->b, m->pb.x, last.add, last.planes, last.rows, m->rms_final, m->pb.xb,
+                                    from.data(), from.size(), dim, m->c.rms_eps));
+        std::vector<float> packed(from.size() < rows.size() ? from.size() * dim : 0);
+        float* to = packed.empty() ? out : packed.data();
+        KRC(m, kr_read(m->b, m->pb.xb, to, from.size() * dim));
+        if (from.size() < rows.size()) {
+            const float* p = packed.data();
+            for (size_t i = 0; i < rows.size(); i++, out += dim) {
+                if (rows[i] < 0)
+                    memset(out, 0, dim * sizeof(float));
+                else
+                    memcpy(out, p, dim * sizeof(float)), p += dim;
+            }
+        }
+        return KR_OK;
+    }
     for (size_t i = 0; i < rows.size(); i++) {
         if (rows[i] < 0) {
             memset(out + i * dim, 0, dim * sizeof(float));
@@ -624,11 +650,18 @@ int krl_prefill(krl_model* m, const size_t* tokens, size_t n, size_t start, floa
     const char* storage = kr_storage(m->b);
     bool batched_in_reference =
         !strcmp(storage, "f32") || !strcmp(storage, "bf16") || !strcmp(storage, "q8_0x4");  // lfm2.rs:489
-    TRY(prefill_rows(m, rows, m->lfm2 && !batched_in_reference));
-    size_t dim = m->c.dim;
-    KRC(m, kr_copy(m->b, m->pb.x, (n - 1) * dim, m->hidden, 0, dim));
-    KRC(m, kr_rms_norm(m->b, m->xb, m->hidden, m->rms_final, 1, dim, m->c.rms_eps));
-    KRC(m, kr_logits(m->b, m->xb, m->logits));
+    LastAdd last;
+    TRY(prefill_rows(m, rows, &last, m->lfm2 && !batched_in_reference));
+    const size_t dim = m->c.dim, end = n - 1;
+    if (last.add != KR_NO_BUF) {
+        KRC(m, kri::norm_quant_from(m->b, m->pb.x, last.add, last.planes, n, m->rms_final, m->pb.xb, &end, 1, dim,
+                                    m->c.rms_eps));
+        KRC(m, kri::logits_q(m->b, m->logits));
+    } else {
+        KRC(m, kr_copy(m->b, m->pb.x, end * dim, m->hidden, 0, dim));
+        KRC(m, kr_rms_norm(m->b, m->xb, m->hidden, m->rms_final, 1, dim, m->c.rms_eps));
+        KRC(m, kr_logits(m->b, m->xb, m->logits));
+    }
     KRC(m, kr_read(m->b, m->logits, m->logits_host.data(), m->c.vocab_size));
     memcpy(logits, m->logits_host.data(), m->c.vocab_size * sizeof(float));
     return KR_OK;
@@ -643,14 +676,15 @@ int krl_decode_batch(krl_model* m, const size_t* tokens, const size_t* rope_pos,
         if (slots[s] >= m->c.seq_len || att_start[s] > slots[s]) return fail(m, "decode_batch row out of range");
         rows.push_back(Row{tokens[s], rope_pos[s], slots[s], att_start[s], 0, 0});
     }
-    TRY(prefill_rows(m, rows));
+    LastAdd last;
+    TRY(prefill_rows(m, rows, &last));
     // the final norm and the classifier over every row (cpu.rs:501-514 per row)
     const size_t vocab = m->c.vocab_size, dim = m->c.dim;
     if (m->batch_logits_rows < n_seq) {
         TRY(alloc(m, n_seq * vocab, &m->batch_logits));
         m->batch_logits_rows = n_seq;
     }
-    KRC(m, kri::norm_quant(m->b, m->pb.x, KR_NO_BUF, 1, m->rms_final, m->pb.xb, n_seq, dim, m->c.rms_eps));
+    KRC(m, kri::norm_quant(m->b, m->pb.x, last.add, last.planes, m->rms_final, m->pb.xb, n_seq, dim, m->c.rms_eps));
     KRC(m, kri::logits_rows(m->b, m->batch_logits, n_seq));
     if (logits) KRC(m, kr_read(m->b, m->batch_logits, logits, n_seq * vocab));
     return KR_OK;
@@ -673,8 +707,9 @@ int krl_prefill_multi(krl_model* m, const size_t* tokens, const size_t* lens, si
         last.push_back((long)rows.size() - 1);
         offset += lens[s];
     }
-    if (!rows.empty()) TRY(prefill_rows(m, rows));
-    return final_hiddens(m, last, hiddens);
+    LastAdd add;
+    if (!rows.empty()) TRY(prefill_rows(m, rows, &add));
+    return final_hiddens(m, last, add, hiddens);
 }
 
 // llama.rs:603-647
@@ -698,8 +733,9 @@ int krl_prefill_shared(krl_model* m, const size_t* prefix, size_t n_prefix, cons
         last.push_back((long)rows.size() - 1);
         base += lens[s];
     }
-    if (!rows.empty()) TRY(prefill_rows(m, rows));
-    return final_hiddens(m, last, hiddens);
+    LastAdd add;
+    if (!rows.empty()) TRY(prefill_rows(m, rows, &add));
+    return final_hiddens(m, last, add, hiddens);
 }
 
 int krl_generate_greedy(krl_model* m, size_t token, size_t pos, size_t n_steps, size_t* out_tokens, int use_graph) {
