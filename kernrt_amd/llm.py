@@ -142,7 +142,7 @@ class Model:
         cols = [np.ascontiguousarray(a, np.uint64) for a in (tokens, rope_pos, slots, att_start)]
         n = len(cols[0])
         assert all(len(c) == n for c in cols)
-        out = np.zeros((n, self.config.vocab_size), np.float32) if read else None
+        out = np.empty((n, self.config.vocab_size), np.float32) if read else None
         self._ck(self.L.krl_decode_batch(self.h, *(_p(c) for c in cols), n, _p(out)))
         return out
 
