@@ -438,15 +438,19 @@ __global__ __launch_bounds__(256, 3) void k_attn_mx_v(float* __restrict__ att, f
     }
     if (__syncthreads_or(vbad) && vwave) {
         // the reference's loop for each element, in position order, over its
-        // own window only: the probabilities from `att`, V from the cache
+        // own window only: the probabilities from `att` (which still holds the
+        // exps where they are not kept), V from the cache
 #pragma unroll
         for (uint32_t v = 0; v < 16; v++) {
             const uint32_t pair = 8 * (v >> 2) + 4 * h + (v & 3);
             const uint32_t n = pair < nr * G ? s_cnt[pair] : 0;
-            const float* prow = att_row(min(pair, nr * G - 1));
+            const uint32_t pc = min(pair, nr * G - 1);
+            const float* prow = att_row(pc);
+            const float sum = psum[(size_t)(r0 + pc / G) * n_heads + h0 + pc % G];
             float acc = 0.0f;
             for (uint32_t i = 0; i < n; i++)
-                acc += prow[i] * vbase[(size_t)win_slot(w0, n_shared, i) * kv_dim + d0 + pr];
+                acc += (keep_att ? prow[i] : div_rn(prow[i], sum)) *
+                       vbase[(size_t)win_slot(w0, n_shared, i) * kv_dim + d0 + pr];
             o[v] = acc;
         }
     }

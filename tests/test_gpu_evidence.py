@@ -22,7 +22,7 @@ import pytest
 
 import kernrt_amd as K
 import oracle as O
-from helpers import assert_bits_equal, product_matrix
+from helpers import assert_bits_equal, gaussian_weights, gpu_model, product_matrix
 
 pytestmark = pytest.mark.gpu
 
@@ -197,6 +197,42 @@ def test_matrix_core_attention_ignores_v_past_a_window(hs):
     width = 16 * hs
     assert np.isfinite(out[:width]).all()
     assert np.isinf(out[width:2 * width]).any()
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hs,rows", [(16, 8, 128, 231), (8, 4, 64, 806)])
+def test_matrix_core_prefill_with_an_infinite_v_row(n_heads, n_kv, hs, rows):
+    # the prompt's last token has infinite values in layer 0; the rows before
+    # it do not read them, and the driver's prefill does not keep the
+    # probabilities. The next call writes the last slot anew, so its logits
+    # show the cache that the earlier rows left in layer 1.
+    dim, bad = 128, 63
+    c = O.Config(dim=dim, hidden_dim=64, n_layers=2, n_heads=n_heads, n_kv_heads=n_kv, vocab_size=64,
+                 seq_len=rows + 8, rms_eps=1e-5, rope_theta=10_000.0, rope_interleaved=False, head_dim=hs)
+    ow = gaussian_weights(c, "q8_0", seed=rows, tied=False)
+    rng = np.random.default_rng(rows)
+    emb = rng.normal(0, 0.02, size=(64, dim)).astype(np.float32)
+    emb[:, 5] = 0.0  # dim 5 belongs to the last token alone: 11.3 once normalized,
+    emb[bad] = 0.0
+    emb[bad, 5] = 1.0
+    ow.set_embedding(O.Matrix(emb, "q8_0"))
+    norm = np.ones(dim, np.float32)
+    norm[5] = 1.5e37  # then 1.7e38,
+    ow.set_norm(0, "att", norm)
+    wv = rng.normal(0, 0.02, size=(c.kv_dim, dim)).astype(np.float32)
+    wv[:, 5] = 0.0
+    wv[3::7, 5] = 100.0  # and past the largest f32 in these dims of v
+    ow.set_proj(0, "v", O.Matrix(wv, "q8_0"))
+    for name, n in (("q", c.q_dim), ("k", c.kv_dim)):
+        w = rng.normal(0, 0.02, size=(n, dim)).astype(np.float32)
+        w[:, 5] = 0.0
+        ow.set_proj(0, name, O.Matrix(w, "q8_0"))
+    prompt = [(7 * i + 1) % 60 for i in range(rows - 1)] + [bad]
+    out = []
+    for m in (gpu_model(c, ow), O.Model(c, ow, "cpu")):
+        assert not m.prefill(prompt, 0).any()  # a row of NaN quantizes to zeros
+        out.append(m.prefill([9], rows - 1))
+    assert np.isfinite(out[1]).all()
+    assert_bits_equal(out[0], out[1], "the token after")
 
 
 # ---- contract checks -----------------------------------------------------------
