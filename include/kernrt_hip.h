@@ -214,7 +214,10 @@ int kr_mfma_rate(kr_ctx* ctx, int kind, size_t workgroups, size_t iters, double*
 /* Launch capture: the ops issued between kr_capture_begin and
  * kr_capture_end are recorded into one HIP graph instead of running (so
  * their inputs must stay alive and unchanged); kr_replay launches that
- * graph `times` times on the context's stream. No counterpart in the
+ * graph `times` times on the context's stream. The graph keeps the context's
+ * workspaces and the row lists (positions, slots, windows) as they were at the
+ * capture, whatever other calls do in between; nothing can be allocated while
+ * the capture is open, so the sequence runs once before it. No counterpart in the
  * reference; it lets a benchmark issue a fixed op sequence the way the
  * model driver's captured decode step does. */
 int kr_capture_begin(kr_ctx* ctx);

@@ -61,6 +61,7 @@ struct IdxStage {
     hipEvent_t ev[2] = {nullptr, nullptr};
     bool recorded[2] = {false, false};
     int cur = 0;
+    bool in_graph = false;  // a kernel of the capture that is open reads it
 };
 
 // The pinned ring of large reads (read_large), a slot made when a read first
@@ -159,10 +160,12 @@ struct kr_ctx {
     // decode attention scratch: scores and per-chunk maxima
     float* attn_scratch = nullptr;
     size_t cap_attn_scratch = 0;
-    // one captured launch sequence (kr_capture_begin / kr_capture_end)
+    // one captured launch sequence (kr_capture_begin / kr_capture_end), and the
+    // memory that its kernels may still use (release), freed with it
     bool capturing = false;
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
+    std::vector<void*> retired, retired_host;
 };
 
 namespace {
@@ -206,77 +209,90 @@ Mat* mat_of(kr_ctx* c, kr_mat m) {
     CHECK(c, name->len >= (size_t)(need), "%s: buffer %u holds %zu elements, needs %zu", #name,   \
           (unsigned)(handle), name->len, (size_t)(need))
 
-int ensure_workspace(kr_ctx* c, size_t rows, size_t k) {
-    size_t nq = rows * k, ns = rows * (k / 32);
-    if (nq > c->cap_q || ns > c->cap_s) c->epoch++;
-    if (nq > c->cap_q) {
-        if (c->wq) HIPCHK(c, hipFree(c->wq));
-        c->wq = nullptr;
-        HIPCHK(c, hipMalloc(&c->wq, nq));
-        c->cap_q = nq;
+// Device memory that the context is done with. A recorded graph keeps what its
+// kernels may point to until the next capture or the context's end; the rest is
+// freed at once (hipFree waits for the device).
+hipError_t release(kr_ctx* c, void* p) {
+    if (!p) return hipSuccess;
+    if (c->capturing || c->graph_exec) {
+        c->retired.push_back(p);
+        return hipSuccess;
     }
-    if (ns > c->cap_s) {
-        if (c->ws) HIPCHK(c, hipFree(c->ws));
-        if (c->wh) HIPCHK(c, hipFree(c->wh));
-        c->ws = nullptr;
-        c->wh = nullptr;
-        HIPCHK(c, hipMalloc(&c->ws, ns * sizeof(float)));
-        HIPCHK(c, hipMalloc(&c->wh, ns * sizeof(uint16_t)));
-        c->cap_s = ns;
+    return hipFree(p);
+}
+
+// *p anew, with room for n elements; null if that fails.
+template <class T>
+int renew(kr_ctx* c, T** p, size_t n) {
+    c->epoch++;
+    T* old = *p;
+    *p = nullptr;
+    HIPCHK(c, release(c, old));
+    HIPCHK(c, hipMalloc(p, n * sizeof(T)));
+    return KR_OK;
+}
+
+// Room for `rows` quantized rows of k in a workspace's three arrays.
+int ensure_rows(kr_ctx* c, size_t rows, size_t k, int8_t** q, float** s, uint16_t** h, size_t* cap_q, size_t* cap_s) {
+    const size_t nq = rows * k, ns = rows * (k / 32);
+    int rc;
+    if (nq > *cap_q) {
+        *cap_q = 0;
+        if ((rc = renew(c, q, nq)) != KR_OK) return rc;
+        *cap_q = nq;
+    }
+    if (ns > *cap_s) {
+        *cap_s = 0;
+        if ((rc = renew(c, s, ns)) != KR_OK) return rc;
+        if ((rc = renew(c, h, ns)) != KR_OK) return rc;
+        *cap_s = ns;
     }
     return KR_OK;
 }
 
+int ensure_workspace(kr_ctx* c, size_t rows, size_t k) {
+    return ensure_rows(c, rows, k, &c->wq, &c->ws, &c->wh, &c->cap_q, &c->cap_s);
+}
+
 static int ensure_workspace2(kr_ctx* c, size_t rows, size_t k) {
-    const size_t nq = rows * k, ns = rows * (k / 32);
-    if (nq > c->cap_q2 || ns > c->cap_s2) c->epoch++;
-    if (nq > c->cap_q2) {
-        if (c->wq2) HIPCHK(c, hipFree(c->wq2));
-        c->wq2 = nullptr;
-        HIPCHK(c, hipMalloc(&c->wq2, nq));
-        c->cap_q2 = nq;
-    }
-    if (ns > c->cap_s2) {
-        if (c->ws2) HIPCHK(c, hipFree(c->ws2));
-        if (c->wh2) HIPCHK(c, hipFree(c->wh2));
-        c->ws2 = nullptr;
-        c->wh2 = nullptr;
-        HIPCHK(c, hipMalloc(&c->ws2, ns * sizeof(float)));
-        HIPCHK(c, hipMalloc(&c->wh2, ns * sizeof(uint16_t)));
-        c->cap_s2 = ns;
-    }
-    return KR_OK;
+    return ensure_rows(c, rows, k, &c->wq2, &c->ws2, &c->wh2, &c->cap_q2, &c->cap_s2);
 }
 
 int ensure_tmp(kr_ctx* c, size_t n) {
     if (n > c->cap_tmp) {
-        c->epoch++;
-        if (c->tmp) HIPCHK(c, hipFree(c->tmp));
-        c->tmp = nullptr;
-        HIPCHK(c, hipMalloc(&c->tmp, n * sizeof(float)));
+        c->cap_tmp = 0;
+        const int rc = renew(c, &c->tmp, n);
+        if (rc) return rc;
         c->cap_tmp = n;
     }
     return KR_OK;
 }
 
 int stage(kr_ctx* c, IdxStage& s, const uint32_t* host, size_t n, const uint32_t** out) {
+    s.in_graph = s.in_graph || c->capturing;
     if (s.dev && s.last.size() == n && memcmp(s.last.data(), host, n * sizeof(uint32_t)) == 0) {
         *out = s.dev;
         return KR_OK;
     }
     if (n > s.cap) {
-        c->epoch++;
-        if (s.dev) HIPCHK(c, hipFree(s.dev));  // hipFree waits for the device
-        s.dev = nullptr;
-        size_t cap = n < 256 ? 256 : n;
-        HIPCHK(c, hipMalloc(&s.dev, cap * sizeof(uint32_t)));
+        const size_t cap = n < 256 ? 256 : n;
+        s.cap = 0;
+        s.last.clear();
+        const int rc = renew(c, &s.dev, cap);
+        if (rc) return rc;
         s.cap = cap;
     }
     if (n > s.pinned_cap) {
+        s.pinned_cap = 0;
         for (int i = 0; i < 2; i++) {
-            if (s.recorded[i]) HIPCHK(c, hipEventSynchronize(s.ev[i]));
-            if (s.pinned[i]) HIPCHK(c, hipHostFree(s.pinned[i]));
+            uint32_t* old = s.pinned[i];
             s.pinned[i] = nullptr;
+            if (old && c->capturing) {  // a recorded copy may read it
+                c->retired_host.push_back(old);
+            } else {
+                if (s.recorded[i]) HIPCHK(c, hipEventSynchronize(s.ev[i]));
+                if (old) HIPCHK(c, hipHostFree(old));
+            }
             s.recorded[i] = false;
         }
         size_t cap = n < 256 ? 256 : n;
@@ -305,6 +321,34 @@ void free_stage(IdxStage& s) {
         if (s.ev[i]) (void)hipEventDestroy(s.ev[i]);
     }
     if (s.dev) (void)hipFree(s.dev);
+}
+
+// The row lists that a capture used stay as its kernels found them: its graph
+// takes their memory over, and the next eager call stages into memory of its own.
+void own_stages(kr_ctx* c) {
+    for (IdxStage* s : {&c->st_pos, &c->st_slots, &c->st_win, &c->st_tok, &c->st_rows}) {
+        if (!s->in_graph) continue;
+        c->epoch++;
+        c->retired.push_back(s->dev);
+        for (int i = 0; i < 2; i++) {
+            c->retired_host.push_back(s->pinned[i]);
+            if (s->ev[i]) (void)hipEventDestroy(s->ev[i]);
+        }
+        *s = IdxStage{};
+    }
+}
+
+void drop_capture(kr_ctx* c) {
+    if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
+    if (c->graph) (void)hipGraphDestroy(c->graph);
+    c->graph_exec = nullptr;
+    c->graph = nullptr;
+    for (void* p : c->retired)
+        if (p) (void)hipFree(p);
+    for (void* p : c->retired_host)
+        if (p) (void)hipHostFree(p);
+    c->retired.clear();
+    c->retired_host.clear();
 }
 
 void free_ring(ReadRing& r) {
@@ -402,7 +446,6 @@ int rope_table(kr_ctx* c, float theta, size_t hs, size_t need_pos, const float2*
     auto key = std::make_pair(kr::f2u(theta), hs);
     RopeTable& t = c->rope[key];
     if (t.n_pos < need_pos) {
-        c->epoch++;
         size_t n_pos = need_pos;
         if (n_pos < c->seq_len) n_pos = c->seq_len;
         if (n_pos < 2 * t.n_pos) n_pos = 2 * t.n_pos;
@@ -415,9 +458,9 @@ int rope_table(kr_ctx* c, float theta, size_t hs, size_t need_pos, const float2*
                 float angle = (float)p * freq[j];
                 host[p * half + j] = make_float2(cosf(angle), sinf(angle));
             }
-        if (t.dev) HIPCHK(c, hipFree(t.dev));
-        t.dev = nullptr;
-        HIPCHK(c, hipMalloc(&t.dev, host.size() * sizeof(float2)));
+        t.n_pos = 0;
+        const int rc = renew(c, &t.dev, host.size());
+        if (rc) return rc;
         HIPCHK(c, hipMemcpy(t.dev, host.data(), host.size() * sizeof(float2), hipMemcpyHostToDevice));
         t.n_pos = n_pos;
     }
@@ -707,8 +750,7 @@ void kr_close(kr_ctx* c) {
         if (p) (void)hipFree(p);
     if (c->t0) (void)hipEventDestroy(c->t0);
     if (c->t1) (void)hipEventDestroy(c->t1);
-    if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
-    if (c->graph) (void)hipGraphDestroy(c->graph);
+    drop_capture(c);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -1020,11 +1062,10 @@ int kr_kv_write(kr_ctx* c, size_t layer, const size_t* slots, kr_buf k, kr_buf v
 // The split-attention scratch (scores and chunk maxima), grown on demand.
 int ensure_attn_scratch(kr_ctx* c, size_t need) {
     if (need > c->cap_attn_scratch) {
-        if (c->attn_scratch) HIPCHK(c, hipFree(c->attn_scratch));  // hipFree waits for the device
-        c->attn_scratch = nullptr;
-        HIPCHK(c, hipMalloc(&c->attn_scratch, need * sizeof(float)));
+        c->cap_attn_scratch = 0;
+        const int rc = renew(c, &c->attn_scratch, need);
+        if (rc) return rc;
         c->cap_attn_scratch = need;
-        c->epoch++;
     }
     return KR_OK;
 }
@@ -1270,11 +1311,8 @@ int kr_stream_read_shape(kr_ctx* c, kr_buf src, size_t offset, size_t len, int c
 
 int kr_capture_begin(kr_ctx* c) {
     CHECK(c, !c->capturing, "a capture is already open");
-    if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
-    if (c->graph) (void)hipGraphDestroy(c->graph);
-    c->graph_exec = nullptr;
-    c->graph = nullptr;
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    drop_capture(c);
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     c->capturing = true;
     return KR_OK;
@@ -1283,7 +1321,9 @@ int kr_capture_begin(kr_ctx* c) {
 int kr_capture_end(kr_ctx* c) {
     CHECK(c, c->capturing, "no capture is open");
     c->capturing = false;
-    HIPCHK(c, hipStreamEndCapture(c->stream, &c->graph));
+    const hipError_t e = hipStreamEndCapture(c->stream, &c->graph);
+    own_stages(c);
+    HIPCHK(c, e);
     HIPCHK(c, hipGraphInstantiate(&c->graph_exec, c->graph, nullptr, nullptr, 0));
     return KR_OK;
 }
