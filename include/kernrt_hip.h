@@ -255,6 +255,12 @@ int kr_dbg_mfma_f32(kr_ctx* ctx, const float* a, const float* b, const float* ac
  * shader clocks each took. No counterpart in the reference. */
 int kr_dbg_serial_sum(kr_ctx* ctx, const float* values, size_t n, size_t count, int waves, uint32_t* out);
 
+/* How often device memory that recorded kernels may point to (workspaces,
+ * scratch, rotation tables, staged row lists) has moved: a graph that a caller
+ * recorded on the stream by other means than kr_capture_begin is valid only
+ * while this stays the same. No counterpart in the reference. */
+uint64_t kr_dbg_epoch(const kr_ctx* ctx);
+
 /* A device matrix as stored: row-major int8 quants [out_dim][in_dim] and the
  * block scales [out_dim][in_dim/32] (f32 for Q8_0, f16 bits for Q8_0x4) --
  * so a host checker can rebuild the reference's Matrix from the very bytes a

@@ -451,6 +451,10 @@ class Hip:
         self._ck(self._L.kr_dbg_mfma_f32(self.ctx, _p(a), _p(b), _p(acc), _p(out), a.shape[0]))
         return out
 
+    def dbg_epoch(self) -> int:
+        """kr_dbg_epoch: how often memory that recorded kernels may hold has moved."""
+        return self._L.kr_dbg_epoch(self.ctx)
+
     def dbg_serial_sum(self, values, waves: int = 1):
         """kr_dbg_serial_sum: values [count, n] summed by the parallel exact
         form over `waves` waves and by the chain -> (fast sums, fast applied,

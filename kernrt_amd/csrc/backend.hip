@@ -1092,8 +1092,10 @@ int stage_windows(kr_ctx* c, const kr_window* windows, size_t n, const kr_attn_s
         w[4 * i + 2] = (uint32_t)x.shared_start;
         w[4 * i + 3] = (uint32_t)x.shared_end;
     }
+    // rows that blocks could take as well take the per-row launches only while their scratch is of moderate size
+    const size_t scratch = n * kr::attention_split_scratch(sp->n_heads, c->seq_len) * sizeof(float);
     out->plan = kr::attention_plan((const kr::DevWindow*)w.data(), n, out->max_count, sp->n_heads, sp->kv_mul,
-                                   sp->head_size);
+                                   sp->head_size, scratch <= (256u << 20));
     w.insert(w.end(), out->plan.blocks.begin(), out->plan.blocks.end());
     return stage(c, c->st_win, w.data(), w.size(), &out->dev);
 }
@@ -1103,10 +1105,14 @@ int attention_many(kr_ctx* c, const float* q, float* out, float* att, size_t lay
                    const kr_attn_spec* sp, int8_t* qo, float* so, uint16_t* ho, bool keep_att = true) {
     const kr::DevWindow* wd = (const kr::DevWindow*)w.dev;
     const float scale = 1.0f / sqrtf((float)sp->head_size);  // cpu.rs:591
-    if (w.plan.kind == kr::ATTN_SPLIT) {
-        int rc = ensure_attn_scratch(
-            c, n * kr::attention_split_scratch(sp->n_heads, kr::attention_split_cap(w.max_count, c->seq_len)));
-        if (rc) return rc;
+    // The per-row launches' scratch holds any window of the cache, so that windows that grow from call to call do
+    // not move it, and is there for few rows whichever launches they take. The matrix-core launches keep each
+    // pair's max and sum in the scratch.
+    const size_t full = n * kr::attention_split_scratch(sp->n_heads, c->seq_len);
+    const bool split = w.plan.kind == kr::ATTN_SPLIT;
+    const int rc = ensure_attn_scratch(c, split || full <= (1u << 20) ? full : 2 * n * sp->n_heads);
+    if (rc) return rc;
+    if (split) {
         HIPCHK(c, kr::launch_attention_split_rows(c->stream, q, out, att, c->kc, c->vc, layer, wd, n, w.max_count,
                                                   sp->n_heads, sp->kv_mul, sp->head_size, sp->kv_dim, sp->seq_len,
                                                   scale, c->attn_scratch, keep_att,
@@ -1115,9 +1121,6 @@ int attention_many(kr_ctx* c, const float* q, float* out, float* att, size_t lay
         if (qo && sp->head_size % 32 != 0) HIPCHK(c, kr::launch_quantize(c->stream, out, n, width, width, qo, so, ho));
         return KR_OK;
     }
-    // the matrix-core prefill attention keeps each pair's max and sum in the scratch
-    int rc = ensure_attn_scratch(c, 2 * n * sp->n_heads);
-    if (rc) return rc;
     HIPCHK(c, kr::launch_attention(c->stream, q, out, att, c->kc, c->vc, layer, wd, n, w.max_count, sp->n_heads,
                                    sp->kv_mul, sp->head_size, sp->kv_dim, sp->seq_len, scale, qo, so, ho, w.plan,
                                    w.dev + 4 * n, c->attn_scratch, keep_att));
@@ -1429,6 +1432,8 @@ int kr_dbg_mfma_f32(kr_ctx* c, const float* a, const float* b, const float* acc,
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return KR_OK;
 }
+
+uint64_t kr_dbg_epoch(const kr_ctx* c) { return c->epoch; }
 
 int kr_dbg_serial_sum(kr_ctx* c, const float* values, size_t n, size_t count, int waves, uint32_t* out) {
     CHECK(c, waves == 1 || waves == 2 || waves == 4 || waves == 16, "waves %d (1, 2, 4 or 16)", waves);

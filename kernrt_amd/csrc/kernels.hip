@@ -2190,9 +2190,8 @@ bool attention_split_rows_ok(size_t max_count, size_t kv_mul, size_t hs) {
     return max_count >= 1 && max_count <= 16384 && (kv_mul * scs + 64 * hs) * sizeof(float) <= kAttnSplitLds;
 }
 
-// The window length that the many-row form's scratch is laid out for: in steps,
-// so that windows that grow by a token a step seldom move it.
-size_t attention_split_cap(size_t max_count, size_t seq_len) {
+// The window length that the many-row form's scratch rows are laid out for.
+static size_t attention_split_cap(size_t max_count, size_t seq_len) {
     return std::min((max_count + 511) & ~(size_t)511, seq_len);
 }
 
@@ -3113,12 +3112,12 @@ static std::vector<uint32_t> attn_blocks(const DevWindow* w, size_t n_rows, size
 // Sequences of their own lengths, blocks by the table: 24 of 700 rows in all,
 // 15/5 heads 19.9 / 30.8, 16/8 heads of 128 108 / 62; 8 of 1500 rows 89 / 247.
 AttnPlan attention_plan(const DevWindow* w, size_t n_rows, size_t max_count, size_t n_heads, size_t kv_mul,
-                        size_t hs) {
+                        size_t hs, bool per_row) {
     AttnPlan p;
     const size_t pairs = n_rows * (n_heads / kv_mul);
-    const bool split = attention_split_rows_ok(max_count, kv_mul, hs);
+    const bool split = attention_split_rows_ok(max_count, kv_mul, hs), choice = split && per_row;
     if (n_rows < 2) {  // k_attention_fast up to 256 positions of small heads (9 against 9.5 us)
-        if (split && (max_count >= 256 || hs == 128)) p.kind = ATTN_SPLIT;
+        if (choice && (max_count >= 256 || hs == 128)) p.kind = ATTN_SPLIT;
         return p;
     }
     auto blocked = [&](size_t R) {  // blocks at least half full, or the regular ones
@@ -3127,9 +3126,9 @@ AttnPlan attention_plan(const DevWindow* w, size_t n_rows, size_t max_count, siz
     };
     const size_t nw = attn_rows_waves(attn_rows_group(kv_mul), hs, max_count);
     if (attention_mx_rows(max_count, kv_mul, hs) && blocked(attention_mx_rows(max_count, kv_mul, hs))) {
-        p.kind = split && pairs <= (hs == 128 ? 1792 : 1280) ? ATTN_SPLIT : ATTN_MX;
+        p.kind = choice && pairs <= (hs == 128 ? 1792 : 1280) ? ATTN_SPLIT : ATTN_MX;
     } else if (nw && blocked(nw * (128 / hs) / attn_rows_group(kv_mul))) {
-        p.kind = split && (hs == 128 || (max_count > 64 && pairs <= 512)) ? ATTN_SPLIT : ATTN_ROWS;
+        p.kind = choice && (hs == 128 || (max_count > 64 && pairs <= 512)) ? ATTN_SPLIT : ATTN_ROWS;
     } else {
         p.kind = split ? ATTN_SPLIT : ATTN_GENERAL;
     }

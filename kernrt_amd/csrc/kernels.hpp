@@ -124,8 +124,10 @@ struct AttnPlan {
     AttnKind kind = ATTN_GENERAL;
     std::vector<uint32_t> blocks;
 };
+// per_row: rows that blocks (or one workgroup per row) could take may take the
+// per-row launches instead; rows that only those can take do so either way.
 AttnPlan attention_plan(const DevWindow* host_windows, size_t n_rows, size_t max_count, size_t n_heads, size_t kv_mul,
-                        size_t hs);
+                        size_t hs, bool per_row);
 hipError_t launch_attention(hipStream_t st, const float* q, float* out, float* att, const float* kc,
                             const float* vc, size_t layer, const DevWindow* windows, size_t n_rows,
                             size_t max_count, size_t n_heads, size_t kv_mul, size_t head_size,
@@ -151,7 +153,6 @@ bool attention_split_ok(size_t max_count, size_t kv_mul, size_t hs);
 // launch_attention_split_rows's geometry check (k_attn_softmax_v_rows).
 bool attention_split_rows_ok(size_t max_count, size_t kv_mul, size_t hs);
 size_t attention_split_scratch(size_t n_heads, size_t seq_len);
-size_t attention_split_cap(size_t max_count, size_t seq_len);
 hipError_t launch_attention_split(hipStream_t st, const float* q, const float* k, const float* v, float* out,
                                   float* att, float* kc, float* vc, size_t layer, const DevWindow* window,
                                   const uint32_t* pos, const float2* table, int interleaved, size_t max_count,
@@ -160,8 +161,7 @@ hipError_t launch_attention_split(hipStream_t st, const float* q, const float* k
                                   const float* knw = nullptr, float eps = 0.0f);
 // The same two launches for many rows with windows of their own (batched
 // decode): q rows already rotated, keys already in the cache; `scratch`
-// holds n_rows * attention_split_scratch(n_heads, attention_split_cap(max_count,
-// seq_len)) floats. keep_att
+// holds n_rows * attention_split_scratch(n_heads, seq_len) floats. keep_att
 // false leaves `att` unwritten; qo/so/ho (head size a multiple of 32) take
 // the output rows' Q8 blocks as well.
 hipError_t launch_attention_split_rows(hipStream_t st, const float* q, float* out, float* att, const float* kc,

@@ -2,8 +2,12 @@
 every window layout gives the oracle's outputs and probabilities bit for bit,
 whichever launches take it."""
 
+import numpy as np
 import pytest
 
+import kernrt_amd as K
+import oracle as O
+from helpers import product_matrix
 from test_gpu_ops import _attention_case
 
 pytestmark = pytest.mark.gpu
@@ -50,3 +54,21 @@ def test_rows_of_one_sequence(n_heads, n_kv, hs, n, start):
 ])
 def test_rows_of_ragged_sequences(n_heads, n_kv, hs, lens, shared):
     _attention_case(shared + sum(lens) + 2, n_heads, n_kv, hs, ragged(lens, shared), sum(lens) + shared)
+
+
+@pytest.mark.parametrize("n,hs", [(1, 64), (1, 128), (6, 64)])
+def test_growing_windows_leave_the_scratch_in_place(n, hs):
+    # a conversation's window grows past 512, 1024, 1536 positions: what the
+    # first call laid out (and a recorded decode step holds) stays
+    hip, seq = K.open("hip"), 2048
+    emb = hip.upload_matrix(product_matrix(O.Matrix(np.ones((8, 32), np.float32), "q8_0")))
+    hip.bind_handles(emb, 0xFFFFFFFF, [{}])
+    hip.prepare(None, K.KvSpec(1, 2 * hs, seq))
+    q, out, att = hip.alloc(n * 4 * hs), hip.alloc(n * 4 * hs), hip.alloc(n * 4 * seq)
+    spec = K.AttnSpec(4, 2, hs, 2 * hs, seq)
+    epochs = []
+    for end in (20, 100, 300, 512, 513, 900, 1025, 1600, 2040):
+        hip.attention(q, out, att, 0, [K.Window(0, end + r, (0, 0)) for r in range(n)], spec)
+        epochs.append(hip.dbg_epoch())
+    assert epochs == epochs[:1] * len(epochs)
+    hip.close()
