@@ -216,8 +216,9 @@ int kr_mfma_rate(kr_ctx* ctx, int kind, size_t workgroups, size_t iters, double*
  * their inputs must stay alive and unchanged); kr_replay launches that
  * graph `times` times on the context's stream. The graph keeps the context's
  * workspaces and the row lists (positions, slots, windows) as they were at the
- * capture, whatever other calls do in between; nothing can be allocated while
- * the capture is open, so the sequence runs once before it. No counterpart in the
+ * capture, whatever other calls do in between. Nothing can be allocated while
+ * the capture is open, so the sequence runs once before it, and the ops of one
+ * capture share their positions, slots and windows. No counterpart in the
  * reference; it lets a benchmark issue a fixed op sequence the way the
  * model driver's captured decode step does. */
 int kr_capture_begin(kr_ctx* ctx);
@@ -254,6 +255,15 @@ int kr_dbg_mfma_f32(kr_ctx* ctx, const float* a, const float* b, const float* ac
  * applied (else the kernels use the chain), the chain's sum bits, and the
  * shader clocks each took. No counterpart in the reference. */
 int kr_dbg_serial_sum(kr_ctx* ctx, const float* values, size_t n, size_t count, int waves, uint32_t* out);
+
+/* Which launches kr_attention takes for n windows, without a device: *kind is
+ * one of KR_ATTN_*. With a block table (irregular blocks of rows that share a
+ * window layout) blocks[0 .. *n_blocks] are the first row of each block, then n
+ * (room for n + 1); else *n_blocks is 0. capturing: as inside a launch capture.
+ * No counterpart in the reference. */
+enum { KR_ATTN_GENERAL = 0, KR_ATTN_ROWS = 1, KR_ATTN_MX = 2, KR_ATTN_SPLIT = 3 };
+int kr_dbg_attention_plan(const kr_window* windows, size_t n, const kr_attn_spec* spec, int capturing, int* kind,
+                          uint32_t* blocks, size_t* n_blocks);
 
 /* How often device memory that recorded kernels may point to (workspaces,
  * scratch, rotation tables, staged row lists) has moved: a graph that a caller

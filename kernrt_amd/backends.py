@@ -150,6 +150,22 @@ def _f32(a) -> np.ndarray:
     return np.ascontiguousarray(a, dtype=np.float32)
 
 
+def attention_plan(windows: Sequence[Window], spec: AttnSpec, capturing: bool = False):
+    """kr_dbg_attention_plan: which launches `attention` takes for these windows,
+    "general", "rows", "mx" or "split", and the first row of each irregular block
+    with the row count behind them ([] for regular blocks or none). No device."""
+    ws = (KrWindow * max(len(windows), 1))(*[KrWindow(w.att_start, w.slot, w.shared[0], w.shared[1])
+                                              for w in windows])
+    s = KrAttnSpec(spec.n_heads, spec.kv_mul, spec.head_size, spec.kv_dim, spec.seq_len)
+    kind, n = C.c_int(), C.c_size_t()
+    blocks = np.zeros(len(windows) + 1, np.uint32)
+    rc = _lib.load().kr_dbg_attention_plan(ws, len(windows), C.byref(s), int(capturing), C.byref(kind), _p(blocks),
+                                           C.byref(n))
+    if rc:
+        raise ValueError(f"no plan for these windows ({rc})")
+    return ("general", "rows", "mx", "split")[kind.value], blocks[:n.value + 1].tolist() if n.value else []
+
+
 def q8_0x4_records(quants: np.ndarray, scales_f16: np.ndarray) -> np.ndarray:
     """The reference's Q8_0x4 storage (`Q8Block4`, quant.rs:113-118) of a
     row-major int8 matrix [out_dim, in_dim] and its f16 scale bits

@@ -1077,25 +1077,42 @@ struct StagedWindows {
     size_t max_count = 0;
     kr::AttnPlan plan;
 };
-int stage_windows(kr_ctx* c, const kr_window* windows, size_t n, const kr_attn_spec* sp, StagedWindows* out) {
-    std::vector<uint32_t> w(4 * n);
+// Which launches n rows take. Rows that blocks could take as well take the
+// per-row launches only while their scratch is of moderate size. In a capture
+// they never do, and blocks come without a table: a replay must not depend on
+// what later row lists left behind, nor the capture on new memory.
+kr::AttnPlan plan_windows(const uint32_t* w, size_t n, size_t max_count, const kr_attn_spec* sp, bool capturing) {
+    const size_t scratch = n * kr::attention_split_scratch(sp->n_heads, sp->seq_len) * sizeof(float);
+    return kr::attention_plan((const kr::DevWindow*)w, n, max_count, sp->n_heads, sp->kv_mul, sp->head_size,
+                              !capturing && scratch <= (256u << 20), !capturing);
+}
+
+int flat_windows(kr_ctx* c, const kr_window* windows, size_t n, size_t seq_len, std::vector<uint32_t>* w,
+                 size_t* max_count) {
+    w->resize(4 * n);
     for (size_t i = 0; i < n; i++) {
         const kr_window& x = windows[i];
-        CHECK(c, x.att_start <= x.slot && x.slot < c->seq_len && x.shared_start <= x.shared_end &&
-                     x.shared_end <= c->seq_len,
+        CHECK(c, x.att_start <= x.slot && x.slot < seq_len && x.shared_start <= x.shared_end && x.shared_end <= seq_len,
               "window %zu out of range", i);
         const size_t count = (x.shared_end - x.shared_start) + x.slot - x.att_start + 1;
-        CHECK(c, count <= c->seq_len, "window %zu attends more than seq_len slots", i);
-        out->max_count = std::max(out->max_count, count);
-        w[4 * i] = (uint32_t)x.att_start;
-        w[4 * i + 1] = (uint32_t)x.slot;
-        w[4 * i + 2] = (uint32_t)x.shared_start;
-        w[4 * i + 3] = (uint32_t)x.shared_end;
+        CHECK(c, count <= seq_len, "window %zu attends more than seq_len slots", i);
+        *max_count = std::max(*max_count, count);
+        (*w)[4 * i] = (uint32_t)x.att_start;
+        (*w)[4 * i + 1] = (uint32_t)x.slot;
+        (*w)[4 * i + 2] = (uint32_t)x.shared_start;
+        (*w)[4 * i + 3] = (uint32_t)x.shared_end;
     }
-    // rows that blocks could take as well take the per-row launches only while their scratch is of moderate size
-    const size_t scratch = n * kr::attention_split_scratch(sp->n_heads, c->seq_len) * sizeof(float);
-    out->plan = kr::attention_plan((const kr::DevWindow*)w.data(), n, out->max_count, sp->n_heads, sp->kv_mul,
-                                   sp->head_size, scratch <= (256u << 20));
+    return KR_OK;
+}
+
+int stage_windows(kr_ctx* c, const kr_window* windows, size_t n, const kr_attn_spec* sp, StagedWindows* out) {
+    std::vector<uint32_t> w;
+    int rc = flat_windows(c, windows, n, c->seq_len, &w, &out->max_count);
+    if (rc) return rc;
+    out->plan = plan_windows(w.data(), n, out->max_count, sp, c->capturing);
+    if (c->capturing && out->plan.kind == kr::ATTN_SPLIT &&
+        n * kr::attention_split_scratch(sp->n_heads, c->seq_len) > c->cap_attn_scratch)
+        out->plan.kind = kr::ATTN_GENERAL;
     w.insert(w.end(), out->plan.blocks.begin(), out->plan.blocks.end());
     return stage(c, c->st_win, w.data(), w.size(), &out->dev);
 }
@@ -1110,7 +1127,7 @@ int attention_many(kr_ctx* c, const float* q, float* out, float* att, size_t lay
     // pair's max and sum in the scratch.
     const size_t full = n * kr::attention_split_scratch(sp->n_heads, c->seq_len);
     const bool split = w.plan.kind == kr::ATTN_SPLIT;
-    const int rc = ensure_attn_scratch(c, split || full <= (1u << 20) ? full : 2 * n * sp->n_heads);
+    const int rc = ensure_attn_scratch(c, split || (full <= (1u << 20) && !c->capturing) ? full : 2 * n * sp->n_heads);
     if (rc) return rc;
     if (split) {
         HIPCHK(c, kr::launch_attention_split_rows(c->stream, q, out, att, c->kc, c->vc, layer, wd, n, w.max_count,
@@ -1430,6 +1447,22 @@ int kr_dbg_mfma_f32(kr_ctx* c, const float* a, const float* b, const float* acc,
     HIPCHK(c, kr::launch_mfma_f32_probe(c->stream, da, db, dc, dout, groups));
     HIPCHK(c, hipMemcpyAsync(out, dout, nc * sizeof(float), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    return KR_OK;
+}
+
+int kr_dbg_attention_plan(const kr_window* windows, size_t n, const kr_attn_spec* sp, int capturing, int* kind,
+                          uint32_t* blocks, size_t* n_blocks) {
+    std::vector<uint32_t> w;
+    size_t max_count = 0;
+    if (n == 0 || sp->kv_mul == 0 || sp->n_heads % sp->kv_mul != 0 || sp->head_size == 0 || sp->head_size > 256 ||
+        sp->head_size % 4 != 0)
+        return KR_ERR_INVALID;
+    int rc = flat_windows(nullptr, windows, n, sp->seq_len, &w, &max_count);
+    if (rc) return rc;
+    const kr::AttnPlan p = plan_windows(w.data(), n, max_count, sp, capturing != 0);
+    *kind = (int)p.kind;
+    *n_blocks = p.blocks.empty() ? 0 : p.blocks.size() - 1;
+    std::copy(p.blocks.begin(), p.blocks.end(), blocks);
     return KR_OK;
 }
 

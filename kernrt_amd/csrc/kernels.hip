@@ -3112,7 +3112,7 @@ static std::vector<uint32_t> attn_blocks(const DevWindow* w, size_t n_rows, size
 // Sequences of their own lengths, blocks by the table: 24 of 700 rows in all,
 // 15/5 heads 19.9 / 30.8, 16/8 heads of 128 108 / 62; 8 of 1500 rows 89 / 247.
 AttnPlan attention_plan(const DevWindow* w, size_t n_rows, size_t max_count, size_t n_heads, size_t kv_mul,
-                        size_t hs, bool per_row) {
+                        size_t hs, bool per_row, bool tables) {
     AttnPlan p;
     const size_t pairs = n_rows * (n_heads / kv_mul);
     const bool split = attention_split_rows_ok(max_count, kv_mul, hs), choice = split && per_row;
@@ -3122,7 +3122,7 @@ AttnPlan attention_plan(const DevWindow* w, size_t n_rows, size_t max_count, siz
     }
     auto blocked = [&](size_t R) {  // blocks at least half full, or the regular ones
         p.blocks = attn_blocks(w, n_rows, R);
-        return p.blocks.empty() || (R > 1 && (p.blocks.size() - 1) * R <= 2 * n_rows);
+        return p.blocks.empty() || (tables && R > 1 && (p.blocks.size() - 1) * R <= 2 * n_rows);
     };
     const size_t nw = attn_rows_waves(attn_rows_group(kv_mul), hs, max_count);
     if (attention_mx_rows(max_count, kv_mul, hs) && blocked(attention_mx_rows(max_count, kv_mul, hs))) {

@@ -126,8 +126,9 @@ struct AttnPlan {
 };
 // per_row: rows that blocks (or one workgroup per row) could take may take the
 // per-row launches instead; rows that only those can take do so either way.
+// tables: irregular blocks may be taken by a table.
 AttnPlan attention_plan(const DevWindow* host_windows, size_t n_rows, size_t max_count, size_t n_heads, size_t kv_mul,
-                        size_t hs, bool per_row);
+                        size_t hs, bool per_row, bool tables);
 hipError_t launch_attention(hipStream_t st, const float* q, float* out, float* att, const float* kc,
                             const float* vc, size_t layer, const DevWindow* windows, size_t n_rows,
                             size_t max_count, size_t n_heads, size_t kv_mul, size_t head_size,

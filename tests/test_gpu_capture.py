@@ -78,3 +78,38 @@ def test_replays_between_eager_calls(windows):
     hip.replay(1)
     assert_bits_equal(hip.read(out, n * q_dim), want, "a second capture")
     hip.close()
+
+
+@pytest.mark.parametrize("warm,wins", [
+    ([(0, 100 + i, 0, 0) for i in range(600)], rows_of([9], 400)),      # one sequence's rows: blocks
+    ([(0, 100 + i, 0, 0) for i in range(600)], rows_of([1], 400)),
+    ([(0, 20 + i, 0, 0) for i in range(40)], rows_of([20, 11, 9], 60)),  # per-row launches without their scratch
+])
+def test_capture_of_windows_that_no_call_had_before(warm, wins):
+    # a capture cannot allocate: it takes the launches that the memory of the
+    # eager calls before it serves
+    rng = np.random.default_rng(len(wins))
+    hip, kv_dim, q_dim, seq = K.open("hip"), KV_HEADS * HS, HEADS * HS, 16384
+    emb = hip.upload_matrix(product_matrix(O.Matrix(np.ones((8, 32), np.float32), "q8_0")))
+    hip.bind_handles(emb, 0xFFFFFFFF, [{}])
+    hip.prepare(None, K.KvSpec(1, kv_dim, seq))
+    for which in (0, 1):
+        hip.kv_upload(which, 0, rng.normal(size=1200 * kv_dim).astype(np.float32))
+    n = max(len(warm), len(wins))
+    q = hip.upload(rng.normal(size=n * q_dim).astype(np.float32))
+    out, att = hip.alloc(n * q_dim), hip.alloc(n * HEADS * seq)
+    spec = K.AttnSpec(HEADS, HEADS // KV_HEADS, HS, kv_dim, seq)
+    wins, warm = ([K.Window(a, s, (c, d)) for a, s, c, d in w] for w in (wins, warm))
+    hip.attention(q, out, att, 0, warm, spec)
+    epoch = hip.dbg_epoch()
+    hip.capture_begin()
+    hip.attention(q, out, att, 0, wins, spec)
+    assert hip.dbg_epoch() == epoch
+    hip.capture_end()
+    hip.replay(1)
+    got = hip.read(out, len(wins) * q_dim)
+    hip.attention(q, out, att, 0, wins, spec)
+    assert_bits_equal(got, hip.read(out, len(wins) * q_dim), "eager")
+    hip.replay(2)
+    assert_bits_equal(got, hip.read(out, len(wins) * q_dim), "again")
+    hip.close()
