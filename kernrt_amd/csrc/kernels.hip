@@ -3111,11 +3111,19 @@ static std::vector<uint32_t> attn_blocks(const DevWindow* w, size_t n_rows, size
 // 200 rows at 100 53 / 42, 250 rows at 0 44 / 43, 128 rows at 1500 214 / 149.
 // Sequences of their own lengths, blocks by the table: 24 of 700 rows in all,
 // 15/5 heads 19.9 / 30.8, 16/8 heads of 128 108 / 62; 8 of 1500 rows 89 / 247.
+// Heads of 128 below the matrix-core windows: a wave of k_attn_rows scores 64
+// positions for all of its block's pairs, so windows this short leave most of
+// its waves idle there, and per row is shorter at any number of rows of several
+// query heads per KV head (sequences of 40-90, 16/8 heads: 250 rows 41 / 30, 2000 rows
+// 346 / 181; 32/8 heads 77 / 39, 677 / 260), and of one up to some 2000 pairs
+// (8/8 heads: 100 rows 21 / 19, 250 rows 37 / 35, 500 rows 55 / 60, 2000 rows
+// 175 / 210).
 AttnPlan attention_plan(const DevWindow* w, size_t n_rows, size_t max_count, size_t n_heads, size_t kv_mul,
                         size_t hs, bool per_row, bool tables) {
     AttnPlan p;
     const size_t pairs = n_rows * (n_heads / kv_mul);
-    const bool split = attention_split_rows_ok(max_count, kv_mul, hs), choice = split && per_row;
+    const bool split = attention_split_rows_ok(max_count, kv_mul, hs);
+    const bool choice = split && per_row && n_rows <= 65535;  // a grid dimension counts the rows
     if (n_rows < 2) {  // k_attention_fast up to 256 positions of small heads (9 against 9.5 us)
         if (choice && (max_count >= 256 || hs == 128)) p.kind = ATTN_SPLIT;
         return p;
@@ -3128,7 +3136,8 @@ AttnPlan attention_plan(const DevWindow* w, size_t n_rows, size_t max_count, siz
     if (attention_mx_rows(max_count, kv_mul, hs) && blocked(attention_mx_rows(max_count, kv_mul, hs))) {
         p.kind = choice && pairs <= (hs == 128 ? 1792 : 1280) ? ATTN_SPLIT : ATTN_MX;
     } else if (nw && blocked(nw * (128 / hs) / attn_rows_group(kv_mul))) {
-        p.kind = choice && (hs == 128 || (max_count > 64 && pairs <= 512)) ? ATTN_SPLIT : ATTN_ROWS;
+        const bool shorter = hs == 128 ? kv_mul > 1 || pairs <= 2048 : max_count > 64 && pairs <= 512;
+        p.kind = choice && shorter ? ATTN_SPLIT : ATTN_ROWS;
     } else {
         p.kind = split ? ATTN_SPLIT : ATTN_GENERAL;
     }

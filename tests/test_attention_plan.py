@@ -72,6 +72,18 @@ def test_large_scratch_is_not_taken_by_choice():
     assert attention_plan(ws, spec(16, 8, 128, 131072))[0] != "split"
 
 
+def test_short_windows_of_128_wide_heads():
+    def equal(n, length):  # sequences of one length: regular blocks
+        return [Window(i // length * length, i) for i in range(n)]
+
+    # one query head per KV head: blocks from 2048 (row, KV head) pairs on
+    assert attention_plan(equal(256, 128), spec(8, 8, 128, 2048))[0] == "split"
+    assert attention_plan(equal(264, 8), spec(8, 8, 128, 2048)) == ("rows", [])
+    assert attention_plan(equal(2000, 40), spec(16, 8, 128, 2048))[0] == "split"
+    # more rows than a grid dimension has workgroups
+    assert attention_plan([Window(0, 0)] * 65536, spec(2, 1, 128, 8))[0] == "rows"
+
+
 def test_refused_windows():
     for w in (Window(5, 4), Window(0, SEQ), Window(0, 1, (3, 2)), Window(0, 1, (0, SEQ + 1)), Window(0, SEQ - 1, (0, 1))):
         with pytest.raises(ValueError):
