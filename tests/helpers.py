@@ -89,6 +89,28 @@ def bits(a) -> np.ndarray:
     return np.ascontiguousarray(a, np.float32).view(np.uint32)
 
 
+def attention_forms(hip, q, n_out, n_att, windows, spec, check):
+    """Layer 0's attention by the launches that an eager call takes for these
+    windows, and inside a launch capture, where rows that blocks can take are
+    taken by blocks: check(out, att) after each. The kinds of launches that ran."""
+    ws = [K.Window(a, s, (x, y)) for a, s, x, y in windows]
+    kinds = []
+    for capturing in (False, True):
+        kind, _ = K.backends.attention_plan(ws, spec, capturing)
+        if kind in kinds:
+            continue
+        kinds.append(kind)
+        out, att = hip.alloc(n_out), hip.alloc(n_att)
+        if capturing:
+            hip.capture_begin()
+        hip.attention(q, out, att, 0, ws, spec)
+        if capturing:
+            hip.capture_end()
+            hip.replay(1)
+        check(hip.read(out, n_out), hip.read(att, n_att))
+    return kinds
+
+
 def assert_bits_equal(got, want, what=""):
     g, w = bits(got), bits(want)
     if not np.array_equal(g, w):

@@ -31,7 +31,8 @@ def ragged(lens, shared=0):
     (15, 5, 64, 255), (15, 5, 64, 256), (32, 32, 64, 700), (16, 8, 128, 3), (32, 16, 128, 2900), (4, 2, 32, 300),
 ])
 def test_one_row(n_heads, n_kv, hs, count):
-    _attention_case(count + 5, n_heads, n_kv, hs, [(2, count + 1, 0, 0)], count)
+    kinds = _attention_case(count + 5, n_heads, n_kv, hs, [(2, count + 1, 0, 0)], count)
+    assert kinds == (["general"] if count == 255 else ["split", "general"])
 
 
 # few rows at long windows: slices of 4 and 16 dims, a workgroup per (row, KV
@@ -39,21 +40,31 @@ def test_one_row(n_heads, n_kv, hs, count):
 @pytest.mark.parametrize("n_heads,n_kv,hs,n,start", [
     (15, 5, 64, 3, 300), (15, 5, 64, 12, 290), (15, 5, 64, 13, 290), (6, 2, 64, 256, 70), (6, 2, 64, 257, 70),
     (4, 4, 64, 30, 800), (16, 8, 128, 2, 150), (16, 8, 128, 30, 150), (16, 8, 128, 225, 3), (8, 8, 32, 65, 60),
+    (16, 1, 128, 9, 130), (12, 2, 128, 9, 130),
 ])
 def test_rows_of_one_sequence(n_heads, n_kv, hs, n, start):
-    _attention_case(start + n + 3, n_heads, n_kv, hs, causal(n, start), n + start)
+    kinds = _attention_case(start + n + 3, n_heads, n_kv, hs, causal(n, start), n + start)
+    by_blocks = (n, start) in ((257, 70), (225, 3), (65, 60)) or n_heads // n_kv in (6, 16)
+    assert kinds[0] in (("rows", "mx") if by_blocks else ("split",)) and kinds[-1] in ("rows", "mx")
 
 
 # sequences whose lengths leave blocks of every size: block tables for
-# k_attn_rows (heads of 64) and for the matrix core (820 and 225 rows), with and
-# without a shared prefix; too ragged for blocks; a row alone at the end
-@pytest.mark.parametrize("n_heads,n_kv,hs,lens,shared", [
-    (15, 5, 64, [1, 5, 6, 37, 64, 3, 2, 1], 0), (15, 5, 64, [70, 33, 48], 9), (4, 4, 64, [7, 50, 1, 9], 20),
-    (6, 2, 64, [1, 1, 2, 1, 1], 0), (16, 8, 128, [100, 30, 66, 1], 0), (16, 8, 128, [180, 17, 1, 15], 12), (16, 8, 128, [180, 17, 1, 30], 12),
-    (4, 2, 64, [790, 30, 1], 0), (8, 4, 32, [40, 3, 25], 7),
+# k_attn_rows and for the matrix core (1, 2, 4 and 8 query heads per workgroup),
+# with and without a shared prefix; too ragged for blocks; a row alone at the end
+@pytest.mark.parametrize("n_heads,n_kv,hs,lens,shared,kind", [
+    (15, 5, 64, [1, 5, 6, 37, 64, 3, 2, 1], 0, "rows"), (15, 5, 64, [70, 33, 48], 9, "rows"),
+    (4, 4, 64, [7, 50, 1, 9], 20, "split"), (6, 2, 64, [1, 1, 2, 1, 1], 0, "split"),
+    (16, 8, 128, [100, 30, 66, 1], 0, "split"), (16, 8, 128, [180, 17, 1, 15], 12, "split"),
+    (16, 8, 128, [180, 17, 1, 30], 12, "mx"), (4, 2, 64, [790, 30, 1], 0, "mx"), (8, 4, 32, [40, 3, 25], 7, "rows"),
+    (8, 8, 128, [90, 60, 40, 30, 44], 0, "rows"), (12, 2, 128, [31, 50, 3], 5, "rows"),
+    (4, 4, 64, [790, 30, 1], 9, "mx"), (16, 4, 128, [300, 120, 60], 4, "mx"), (16, 2, 64, [790, 30, 1], 0, "mx"),
 ])
-def test_rows_of_ragged_sequences(n_heads, n_kv, hs, lens, shared):
-    _attention_case(shared + sum(lens) + 2, n_heads, n_kv, hs, ragged(lens, shared), sum(lens) + shared)
+def test_rows_of_ragged_sequences(n_heads, n_kv, hs, lens, shared, kind):
+    wins = ragged(lens, shared)
+    kinds = _attention_case(shared + sum(lens) + 2, n_heads, n_kv, hs, wins, sum(lens) + shared)
+    spec = K.AttnSpec(n_heads, n_heads // n_kv, hs, n_kv * hs, shared + sum(lens) + 2)
+    _, blocks = K.backends.attention_plan([K.Window(a, s, (x, y)) for a, s, x, y in wins], spec)
+    assert kinds[0] == kind and bool(blocks) == (kind != "split")
 
 
 @pytest.mark.parametrize("n,hs", [(1, 64), (1, 128), (6, 64)])
