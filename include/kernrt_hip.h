@@ -265,6 +265,12 @@ enum { KR_ATTN_GENERAL = 0, KR_ATTN_ROWS = 1, KR_ATTN_MX = 2, KR_ATTN_SPLIT = 3 
 int kr_dbg_attention_plan(const kr_window* windows, size_t n, const kr_attn_spec* spec, int capturing, int* kind,
                           uint32_t* blocks, size_t* n_blocks);
 
+/* At most this many pinned slots (of 2 MiB) and worker threads for each of the
+ * context's large reads (up to 8 each, as it starts): what a read finds where
+ * pinned memory or threads run out. With none of either a large read is one
+ * pageable copy. No counterpart in the reference. */
+int kr_dbg_read_limits(kr_ctx* ctx, size_t slots, size_t threads);
+
 /* How often device memory that recorded kernels may point to (workspaces,
  * scratch, rotation tables, staged row lists) has moved: a graph that a caller
  * recorded on the stream by other means than kr_capture_begin is valid only

@@ -106,6 +106,7 @@ _SIGS = {
     "kr_dbg_block_dots": (i32, [vp, u32, u32, sz, vp]),
     "kr_dbg_mfma_f32": (i32, [vp, vp, vp, vp, vp, sz]),
     "kr_dbg_attention_plan": (i32, [vp, sz, vp, i32, vp, vp, vp]),
+    "kr_dbg_read_limits": (i32, [vp, sz, sz]),
     "kr_dbg_epoch": (C.c_uint64, [vp]),
     "kr_dbg_serial_sum": (i32, [vp, vp, sz, sz, i32, vp]),
     "kr_kv_upload": (i32, [vp, i32, sz, vp, sz]),

@@ -467,6 +467,10 @@ class Hip:
         self._ck(self._L.kr_dbg_mfma_f32(self.ctx, _p(a), _p(b), _p(acc), _p(out), a.shape[0]))
         return out
 
+    def dbg_read_limits(self, slots: int, threads: int):
+        """kr_dbg_read_limits: at most so many pinned slots and workers for a large read."""
+        self._ck(self._L.kr_dbg_read_limits(self.ctx, slots, threads))
+
     def dbg_epoch(self) -> int:
         """kr_dbg_epoch: how often memory that recorded kernels may hold has moved."""
         return self._L.kr_dbg_epoch(self.ctx)

@@ -11,14 +11,17 @@
 #include <math.h>
 #include <stdarg.h>
 #include <stdio.h>
+#include <sched.h>
 #include <string.h>
 
 #include <algorithm>
 #include <array>
 #include <atomic>
+#include <condition_variable>
 #include <exception>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <utility>
@@ -64,12 +67,11 @@ struct IdxStage {
     bool in_graph = false;  // a kernel of the capture that is open reads it
 };
 
-// The pinned ring of large reads (read_large), a slot made when a read first
-// gets to it: pinning all 16 MiB took 0.8 ms of a context's first read.
-struct ReadRing {
-    static constexpr size_t kSlots = 8, kSlot = 2 << 20;
-    uint8_t* slot[kSlots] = {};
-    hipEvent_t ev[kSlots] = {};
+// A pinned piece of large reads (read_large) and the event behind its copy.
+struct ReadSlot {
+    static constexpr size_t kBytes = 2 << 20;
+    uint8_t* p = nullptr;
+    hipEvent_t ev = nullptr;
 };
 
 struct RopeTable {
@@ -146,7 +148,7 @@ struct kr_ctx {
     float* tmp = nullptr;
     size_t cap_tmp = 0;
     IdxStage st_pos, st_slots, st_win, st_tok, st_rows;
-    ReadRing read_ring;
+    size_t read_slots = 8, read_threads = 8;  // at most, for one large read
     std::map<std::pair<uint32_t, size_t>, RopeTable> rope;
     uint32_t* tokens = nullptr;
     static constexpr size_t kTokens = 1 << 16;
@@ -351,90 +353,191 @@ void drop_capture(kr_ctx* c) {
     c->retired_host.clear();
 }
 
-void free_ring(ReadRing& r) {
-    for (size_t i = 0; i < ReadRing::kSlots; i++) {
-        if (r.ev[i]) (void)hipEventDestroy(r.ev[i]);
-        if (r.slot[i]) (void)hipHostFree(r.slot[i]);
+// The pinned slots that no read is using, shared by the contexts of the process:
+// the host's first touch of a new slot faults in its 512 pages, 0.8 ms and more
+// where a new context's read had to. At most kKeep for each device, freed with
+// the last context.
+class SlotPool {
+  public:
+    void open() {
+        std::lock_guard<std::mutex> l(m_);
+        contexts_++;
     }
-    r = ReadRing{};
+    void close() {
+        std::lock_guard<std::mutex> l(m_);
+        if (--contexts_ == 0) {
+            for (auto& d : idle_) destroy(d.second);
+            idle_.clear();
+        }
+    }
+    // n slots, or as many as there is pinned memory for
+    std::vector<ReadSlot> take(int device, size_t n) {
+        std::vector<ReadSlot> out;
+        out.reserve(n);
+        {
+            std::lock_guard<std::mutex> l(m_);
+            std::vector<ReadSlot>& v = idle_[device];
+            for (; out.size() < n && !v.empty(); v.pop_back()) out.push_back(v.back());
+        }
+        while (out.size() < n) {
+            ReadSlot s;
+            if (hipHostMalloc((void**)&s.p, ReadSlot::kBytes) != hipSuccess ||
+                hipEventCreateWithFlags(&s.ev, hipEventDisableTiming) != hipSuccess) {
+                if (s.p) (void)hipHostFree(s.p);
+                (void)hipGetLastError();  // not the next launch's
+                break;
+            }
+            out.push_back(s);
+        }
+        return out;
+    }
+    // no copy into them is under way
+    void give(int device, std::vector<ReadSlot>& slots) {
+        std::lock_guard<std::mutex> l(m_);
+        std::vector<ReadSlot>& v = idle_[device];
+        v.reserve(kKeep);
+        for (; v.size() < kKeep && !slots.empty(); slots.pop_back()) v.push_back(slots.back());
+        destroy(slots);
+    }
+    static void destroy(std::vector<ReadSlot>& slots) {
+        for (ReadSlot& s : slots) {
+            (void)hipEventDestroy(s.ev);
+            (void)hipHostFree(s.p);
+        }
+        slots.clear();
+    }
+
+  private:
+    static constexpr size_t kKeep = 8;
+    std::mutex m_;
+    std::map<int, std::vector<ReadSlot>> idle_;
+    size_t contexts_ = 0;
+};
+
+SlotPool& slot_pool() {
+    static SlotPool* pool = new SlotPool;  // contexts may be closed as late as at exit
+    return *pool;
 }
 
-hipError_t ensure_slot(ReadRing& r, size_t i) {
-    if (!r.ev[i]) {
-        const hipError_t e = hipEventCreateWithFlags(&r.ev[i], hipEventDisableTiming);
-        if (e != hipSuccess) return e;
-    }
-    return r.slot[i] ? hipSuccess : hipHostMalloc((void**)&r.slot[i], ReadRing::kSlot);
+size_t usable_cores() {
+    cpu_set_t set;
+    CPU_ZERO(&set);
+    return sched_getaffinity(0, sizeof set, &set) == 0 ? std::max(CPU_COUNT(&set), 1) : 1;
 }
 
-// From this many bytes on a read goes through read_large. 64 x 151936 logits,
-// 39 MB, read into fresh pages after 2.0 ms of kernels: 4.9-6 ms in all as one
-// pageable copy, whose single host thread also takes every page fault.
+// From this many bytes on a read goes through read_large: us as one pageable copy
+// (whose one thread also takes every page fault) / through slots, warm, 4 MiB 278
+// / 265, 6 MiB 358 / 269, 12 MiB 716 / 452, 20 MiB 1186 / 667, 39 MiB 4138 / 1202;
+// the first of a new context 4 MiB 595 / 608, 12 MiB 1778 / 1473, 39 MiB 5211 /
+// 3658. The host's CPU time in such a read is that of 1.5 to 2 threads.
 constexpr size_t kReadLarge = 4 << 20;
 
-// The barrier read of many bytes: worker threads fault the destination's pages
-// in while the kernels before the read still run, then copy each slot of the
-// pinned ring out as the device fills it. The workers end with the call.
-int read_large(kr_ctx* c, const uint8_t* src, uint8_t* out, size_t bytes) {
-    ReadRing& ring = c->read_ring;
-    constexpr size_t S = ReadRing::kSlots, B = ReadRing::kSlot;
-    const size_t chunks = (bytes + B - 1) / B;
-    std::vector<std::atomic<int>> state(chunks);  // 0 waiting, 1 its copy and event are issued, 2 copied out
+// The copies of read_large. This thread issues them and waits for their events,
+// as it would for one copy; worker threads, which make no HIP call and end with
+// the read, fault the destination's pages in while the kernels before it still
+// run, then sleep until a slot is full and copy it out. False: not all of it.
+bool read_through(kr_ctx* c, const uint8_t* src, uint8_t* out, size_t bytes, const std::vector<ReadSlot>& slots) {
+    constexpr size_t B = ReadSlot::kBytes;
+    const size_t S = slots.size(), chunks = (bytes + B - 1) / B;
+    const size_t want = std::min({c->read_threads, chunks, usable_cores()});
     std::vector<std::atomic<int>> pages(chunks);  // 0 as they came, 1 being faulted in, 2 done, 3 left to the copy
-    for (size_t i = 0; i < chunks; i++) state[i].store(0), pages[i].store(0);
-    std::atomic<size_t> next{0}, touch{0};
-    std::atomic<int> stop{0};  // an error code of HIP's; the others leave as they see it
+    for (std::atomic<int>& p : pages) p.store(0);
+    std::vector<char> copied(chunks, 0);
+    std::vector<std::thread> pool;
+    pool.reserve(want);
+    std::atomic<size_t> next{0}, touch{0}, ready{0};
+    std::mutex m;  // copied and stop, and ready where it is waited for
+    std::condition_variable full, empty;
+    bool stop = false;
     auto work = [&] {
-        (void)hipSetDevice(c->device);
         for (size_t i; (i = next.fetch_add(1)) < chunks;) {
-            const auto issued = [&] { return state[i].load(std::memory_order_acquire) == 1; };
-            while (!(issued() && hipEventQuery(ring.ev[i % S]) == hipSuccess)) {  // the pages meanwhile
+            while (ready.load(std::memory_order_acquire) <= i) {
                 const size_t j = touch.fetch_add(1);
                 if (j >= chunks) break;
                 if (pages[j].exchange(1) != 0) continue;  // its copy is under way
                 for (size_t p = j * B; p < std::min(bytes, (j + 1) * B); p += 4096) ((volatile uint8_t*)out)[p] = 0;
                 pages[j].store(2, std::memory_order_release);
             }
-            while (!issued()) {
-                if (stop.load()) return;
-                std::this_thread::yield();
-            }
-            const hipError_t e = hipEventSynchronize(ring.ev[i % S]);
-            if (e != hipSuccess) {
-                stop.store((int)e);
-                return;
+            {
+                std::unique_lock<std::mutex> l(m);
+                full.wait(l, [&] { return stop || ready.load() > i; });
+                if (ready.load() <= i) return;
             }
             if (pages[i].exchange(3) == 1)  // being faulted in by another worker, which ends with a 2
                 while (pages[i].load(std::memory_order_acquire) != 2) std::this_thread::yield();
-            memcpy(out + i * B, ring.slot[i % S], std::min(B, bytes - i * B));
-            state[i].store(2, std::memory_order_release);
+            memcpy(out + i * B, slots[i % S].p, std::min(B, bytes - i * B));
+            {
+                std::lock_guard<std::mutex> l(m);
+                copied[i] = 1;
+            }
+            empty.notify_one();
         }
     };
-    std::vector<std::thread> pool;
+    size_t issued = 0;
+    auto issue = [&] {
+        const ReadSlot& s = slots[issued % S];
+        const size_t at = issued++ * B;
+        return hipMemcpyAsync(s.p, src + at, std::min(B, bytes - at), hipMemcpyDeviceToHost, c->stream) == hipSuccess &&
+               hipEventRecord(s.ev, c->stream) == hipSuccess;
+    };
+    while (issued < std::min(S, chunks))
+        if (!issue()) return false;
     try {
-        const size_t want = std::min<size_t>(8, chunks);
-        pool.reserve(want);
         while (pool.size() < want) pool.emplace_back(work);
     } catch (const std::exception&) {
         // as many workers as the system gives
     }
-    hipError_t e = pool.empty() ? hipErrorOutOfMemory : hipSuccess;
-    for (size_t i = 0; i < chunks && e == hipSuccess; i++) {
-        while (i >= S && state[i - S].load(std::memory_order_acquire) != 2 && !stop.load()) std::this_thread::yield();
-        if (stop.load()) break;
-        e = ensure_slot(ring, i % S);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(ring.slot[i % S], src + i * B, std::min(B, bytes - i * B), hipMemcpyDeviceToHost,
-                               c->stream);
-        if (e == hipSuccess) e = hipEventRecord(ring.ev[i % S], c->stream);
-        if (e == hipSuccess) state[i].store(1, std::memory_order_release);
+    bool ok = !pool.empty();
+    for (size_t i = 0; ok && i < chunks;) {
+        size_t next_free = issued;  // chunks up to here have an empty slot
+        if (issued < chunks) {
+            std::unique_lock<std::mutex> l(m);
+            if (i == issued) empty.wait(l, [&] { return copied[issued - S]; });
+            while (next_free < chunks && copied[next_free - S]) next_free++;
+        }
+        while (ok && issued < next_free) ok = issue();
+        if (!ok || i == issued) continue;
+        ok = hipEventSynchronize(slots[i % S].ev) == hipSuccess;
+        {
+            std::lock_guard<std::mutex> l(m);
+            ready.store(ok ? ++i : i);
+        }
+        full.notify_all();
     }
-    if (e != hipSuccess) stop.store((int)e);
+    {
+        std::lock_guard<std::mutex> l(m);
+        stop = !ok;
+    }
+    full.notify_all();
     for (std::thread& t : pool) t.join();
-    if (stop.load()) {  // no thread, no pinned memory, or an error that the plain copy meets again
-        (void)hipGetLastError();
-        HIPCHK(c, hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, c->stream));
+    return ok;
+}
+
+// The barrier read of many bytes, through pinned slots; as one pageable copy
+// where there is no pinned memory, no thread, or an error (which it meets again).
+int read_large(kr_ctx* c, const uint8_t* src, uint8_t* out, size_t bytes) {
+    bool whole = false;
+    hipError_t e = hipSuccess;
+    try {
+        const size_t chunks = (bytes + ReadSlot::kBytes - 1) / ReadSlot::kBytes;
+        std::vector<ReadSlot> slots = slot_pool().take(c->device, std::min(chunks, c->read_slots));
+        try {
+            whole = !slots.empty() && read_through(c, src, out, bytes, slots);
+        } catch (const std::bad_alloc&) {
+        }
+        e = hipStreamSynchronize(c->stream);  // no slot is written any more
+        if (e == hipSuccess)
+            slot_pool().give(c->device, slots);
+        else
+            SlotPool::destroy(slots);
+    } catch (const std::bad_alloc&) {
     }
+    if (whole) {
+        HIPCHK(c, e);
+        return KR_OK;
+    }
+    (void)hipGetLastError();
+    HIPCHK(c, hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return KR_OK;
 }
@@ -709,6 +812,7 @@ int kr_open(int device, kr_ctx** out, char* detail, size_t detail_len) {
         return KR_ERR_NO_DEVICE;
     }
     kr_ctx* c = new kr_ctx();
+    slot_pool().open();
     c->device = device;
     c->devname = prop.name[0] ? prop.name : prop.gcnArchName;
     if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
@@ -743,7 +847,6 @@ void kr_close(kr_ctx* c) {
     free_stage(c->st_win);
     free_stage(c->st_tok);
     free_stage(c->st_rows);
-    free_ring(c->read_ring);
     void* ptrs[] = {c->kc, c->vc, c->wq, c->ws, c->wh, c->wq2, c->ws2, c->wh2, c->tmp, c->tokens, c->counter,
                     c->attn_scratch};
     for (void* p : ptrs)
@@ -752,6 +855,7 @@ void kr_close(kr_ctx* c) {
     if (c->t1) (void)hipEventDestroy(c->t1);
     drop_capture(c);
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    slot_pool().close();
     delete c;
 }
 
@@ -1463,6 +1567,12 @@ int kr_dbg_attention_plan(const kr_window* windows, size_t n, const kr_attn_spec
     *kind = (int)p.kind;
     *n_blocks = p.blocks.empty() ? 0 : p.blocks.size() - 1;
     std::copy(p.blocks.begin(), p.blocks.end(), blocks);
+    return KR_OK;
+}
+
+int kr_dbg_read_limits(kr_ctx* c, size_t slots, size_t threads) {
+    c->read_slots = std::min<size_t>(slots, 8);
+    c->read_threads = std::min<size_t>(threads, 8);
     return KR_OK;
 }
 
