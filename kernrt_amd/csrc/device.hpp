@@ -165,11 +165,12 @@ __device__ __forceinline__ void rope_out(const RopeOut& ro, int mi, float* q, ui
     dst[32] = r1;
 }
 
-// The four-partial Q8_0 GEMM (gemm.hip) over a matrix set, rows >= 8.
+// The GEMM over a matrix set with either epilogue, any row count: the four
+// partial sums of Q8_0 or the FMA chain of Q8_0x4, direct or by tiles (gemm.hip).
 hipError_t launch_gemm_q8(hipStream_t st, int sem, const MatSet& ms, size_t k, QuantAct x, size_t rows,
                           int32_t* dbg);
-// The same for either epilogue and any row count, every wave staging its own
-// operands (gemm_direct.hip): few rows or narrow outputs. _swi and _rope: the
+// Its direct form, every wave staging its own operands (gemm_direct.hip): few
+// rows or narrow outputs. _swi and _rope: the
 // gate/up and q/k/v launches with their epilogues.
 hipError_t launch_gemm_direct(hipStream_t st, int sem, const MatSet& ms, size_t k, QuantAct x, size_t rows,
                               int32_t* dbg);
@@ -178,10 +179,17 @@ hipError_t launch_direct_rope(hipStream_t st, int sem, const MatSet& ms, size_t 
                               RopeOut ro);
 // The Q8_0x4 forms by grid: direct up to kDirectTiles16 16x16 units (one wave
 // each), then 64x64 tiles (a 32x32 unit per wave) up to kChainTiles64 of them,
-// then 128x128 tiles (32x64 per wave).
+// then 128x128 tiles (32x64 per wave). The two forms with an epilogue count
+// workgroups of four 16x16 units. us, direct / 64x64 tiles, Q8_0x4:
+//   SiLU  2560x960: 240 workgroups 8.7 / 12.4, 320 10.5 / 13.0, 480 10.7 / 13.1, 560 13.9 / 13.1
+//         4608x1536: 144 8.7 / 15.1, 432 13.2 / 15.7, 576 17.3 / 16.4; 8192x2048: 256 11 / 18, 512 16 / 17, 768 21 / 18
+//   RoPE  1600x960: 200 7.2 / 13.0, 400 9.9 / 13.8, 625 13.3 / 13.4
+//         6144x2048: 192 10.0 / 15.8, 384 14.3 / 18.4, 480 14.5 / 18.4, 576 19.7 / 18.2
+// Both cross near two workgroups per CU (512). The RoPE line lies below that at
+// 400, the SiLU line at one per CU, where direct is well ahead.
 static constexpr size_t kDirectTiles16 = 1408, kChainTiles64 = 640, kDirectSwiMax = 256, kDirectRopeMax = 400;
 
-// The chunk pipeline shared by both GEMM kernels. At chunk c, the register
+// The chunk pipeline of k_gemm_q8_s16 (gemm.hip). At chunk c, the register
 // stage (c + 1) % NS holds chunk c + 1 and LDS buffer c & 1 holds chunk c.
 // The chunk count is padded to a multiple of NS and every load and store is
 // unconditional (loads clamp to the last chunk, compute skips blocks past

@@ -31,8 +31,8 @@ typedef float d_v16f __attribute__((ext_vector_type(16)));
 
 enum { EPI_PLAIN = 0, EPI_SWI = 1, EPI_ROPE = 2 };
 
-// Four waves side by side: a workgroup's tile is 16 rows x 64 columns.
-// EPI_SWI: columns 0..31 are gate rows, 32..63 up rows of hidden block nt;
+// NW waves side by side: a workgroup's tile is 16 rows x 16 NW columns, of one
+// wave in the plain form, of four with an epilogue. EPI_SWI: columns 0..31 are gate rows, 32..63 up rows of hidden block nt;
 // EPI_ROPE: the 64 columns are one head.
 template <int SEM, int EPI, int NW, int NS, bool DBG>
 __global__ __launch_bounds__(64 * NW) void k_gemm_direct(MatSet ms, QuantAct x, uint32_t M, uint32_t K, uint32_t mtiles,
@@ -215,7 +215,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_direct(MatSet ms, QuantAct x, 
     }
 }
 
-// Fill in the tile counts (64 columns) and launch over 16-row tiles.
+// Fill in the tile counts (16 NW columns) and launch over 16-row tiles.
 template <int SEM, int EPI, int NW, int NS>
 static hipError_t direct_go(hipStream_t st, MatSet ms, QuantAct x, size_t rows, size_t k, int32_t* dbg, SwiOut so,
                             RopeOut ro) {

@@ -67,19 +67,11 @@ hipError_t launch_qk_norm_rope_kv(hipStream_t st, float* q, float* k, const floa
                                   size_t head_size, int interleaved, float* kc, float* vc, size_t layer,
                                   size_t seq_len);
 
-// y[m*ldy + n] for m < rows. Uses the GEMV path (rows <= 4) or the MFMA GEMM.
-// One decode row (M = 1) of 1-3 projections with the producer of their input
-// fused in front: pro_kind 1 = x (+= add) -> rms_norm(w, eps) -> Q8 (the
-// updated x row goes to x_out when non-null), 3 = Q8 of the f32 row a (which
-// also goes to (q, s, h) when q is non-null).
 // One decode row of gate/up with the producer in front (x (+= add) ->
 // rms_norm(norm_w, eps) -> Q8, the updated x row to x_out when non-null) and
 // h = silu(gate) * up behind, quantized into (hq, hs, hh) for the down
 // projection; h itself goes to hf when non-null. Needs swiglu_fusable.
 bool swiglu_fusable(const DevMatrix& gate, const DevMatrix& up);
-// Prefill gate/up of Q8_0 matrices with SiLU(gate) * up and its Q8 blocks as
-// the GEMM's epilogue: h's quants / f32 scales / f16 scale bits [rows][n]
-// from the quantized rows x (one launch for gate/up + silu_quant).
 // The chain-split Q8_0 GEMM (gemm.hip): `cm` is a chain-major copy (launch_chain_major),
 // x chain-major too; y4 receives the four partial-sum planes [4][rows][cm.n].
 hipError_t launch_chain_major(hipStream_t st, const DevMatrix& m, int8_t* cq, float* cs);
@@ -91,14 +83,23 @@ hipError_t launch_qkv_rope(hipStream_t st, const DevMatrix& q, const DevMatrix& 
                               size_t rows, float* yq, const uint32_t* pos, const uint32_t* slots, const float2* tab,
                               float* kc, float* vc);
 hipError_t launch_gemm_q8_cs(hipStream_t st, const DevMatrix& cm, QuantAct x, size_t rows, float* y4);
+// Gate/up of a batch with SiLU(gate) * up and its Q8 blocks as the GEMM's
+// epilogue: h's quants / f32 scales / f16 scale bits [rows][n] from the quantized
+// rows x (one launch for gate/up + silu_quant).
 hipError_t launch_gate_up_silu(hipStream_t st, const DevMatrix& gate, const DevMatrix& up, QuantAct x, size_t rows,
                                   int8_t* hq, float* hs, uint16_t* hh, bool chain_major = false);
 hipError_t launch_gate_up_swiglu(hipStream_t st, int sem, const DevMatrix& gate, const DevMatrix& up, const float* x,
                                  const float* add, const float* norm_w, float* x_out, float eps, int8_t* hq,
                                  float* hs, uint16_t* hh, float* hf);
+// One decode row (M = 1) of 1-3 projections with the producer of their input
+// fused in front: pro_kind 1 = x (+= add) -> rms_norm(w, eps) -> Q8 (the
+// updated x row goes to x_out when non-null), 3 = Q8 of the f32 row a (which
+// also goes to (q, s, h) when q is non-null).
 hipError_t launch_project_pro(hipStream_t st, int sem, const DevMatrix* const* w, float* const* y, int count,
                               int pro_kind, const float* a, const float* b, const float* norm_w, float* x_out,
                               float eps, int8_t* q = nullptr, float* s = nullptr, uint16_t* h = nullptr);
+// y[m*ldy + n] for m < rows: GEMV passes of up to four rows, or the GEMM on the
+// matrix core from gemm_min_rows rows (5 or 8).
 hipError_t launch_project(hipStream_t st, int sem, const DevMatrix& w, QuantAct x, size_t rows,
                           float* y, size_t ldy, int32_t* dbg_block_dots);
 
@@ -147,11 +148,10 @@ hipError_t launch_attention_mx(hipStream_t st, const float* q, float* out, float
                                bool keep_att, const uint32_t* blocks, size_t n_blocks);
 // Decode attention of one row in two launches (scores by 64-row chunks with
 // RoPE and the kv_write of k/v folded in, and the per-head q / k RMSNorm
-// where qnw / knw are given, then softmax + V by head slices of 4 dims);
-// `scratch` holds
-// attention_split_scratch(n_heads, seq_len) floats.
+// where qnw / knw are given, then softmax + V by head slices of 4 or 16 dims);
+// `scratch` holds attention_split_scratch(n_heads, seq_len) floats.
 bool attention_split_ok(size_t max_count, size_t kv_mul, size_t hs);
-// launch_attention_split_rows's geometry check (k_attn_softmax_v_rows).
+// launch_attention_split_rows's geometry check.
 bool attention_split_rows_ok(size_t max_count, size_t kv_mul, size_t hs);
 size_t attention_split_scratch(size_t n_heads, size_t seq_len);
 hipError_t launch_attention_split(hipStream_t st, const float* q, const float* k, const float* v, float* out,
@@ -160,8 +160,9 @@ hipError_t launch_attention_split(hipStream_t st, const float* q, const float* k
                                   size_t n_heads, size_t kv_mul, size_t hs, size_t kv_dim, size_t seq_len,
                                   float scale, float* scratch, const float* qnw = nullptr,
                                   const float* knw = nullptr, float eps = 0.0f);
-// The same two launches for many rows with windows of their own (batched
-// decode): q rows already rotated, keys already in the cache; `scratch`
+// The same two launches for one or many rows with windows of their own: q rows
+// already rotated, keys already in the cache, softmax + V by slices of 4 or 16
+// dims or a workgroup per (row, KV head) (attn_slice_dims); `scratch`
 // holds n_rows * attention_split_scratch(n_heads, seq_len) floats. keep_att
 // false leaves `att` unwritten; qo/so/ho (head size a multiple of 32) take
 // the output rows' Q8 blocks as well.
