@@ -340,6 +340,13 @@ void own_stages(kr_ctx* c) {
     }
 }
 
+// Before a capture, with the stream idle: a captured copy need not wait for the
+// eager ones (nor may it, for events of the stream that captures).
+void settle_stages(kr_ctx* c) {
+    for (IdxStage* s : {&c->st_pos, &c->st_slots, &c->st_win, &c->st_tok, &c->st_rows})
+        s->recorded[0] = s->recorded[1] = false;
+}
+
 void drop_capture(kr_ctx* c) {
     if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
     if (c->graph) (void)hipGraphDestroy(c->graph);
@@ -1436,6 +1443,7 @@ int kr_stream_read_shape(kr_ctx* c, kr_buf src, size_t offset, size_t len, int c
 int kr_capture_begin(kr_ctx* c) {
     CHECK(c, !c->capturing, "a capture is already open");
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    settle_stages(c);
     drop_capture(c);
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     c->capturing = true;
