@@ -2190,11 +2190,6 @@ bool attention_split_rows_ok(size_t max_count, size_t kv_mul, size_t hs) {
     return max_count >= 1 && max_count <= 16384 && (kv_mul * scs + 64 * hs) * sizeof(float) <= kAttnSplitLds;
 }
 
-// The window length that the many-row form's scratch rows are laid out for.
-static size_t attention_split_cap(size_t max_count, size_t seq_len) {
-    return std::min((max_count + 511) & ~(size_t)511, seq_len);
-}
-
 // scores [n_heads][round4(seq_len)] | chunk maxima [n_heads][attn_split_ms(seq_len)]
 size_t attention_split_scratch(size_t n_heads, size_t seq_len) {
     return n_heads * (((seq_len + 3) & ~(size_t)3) + attn_split_ms(seq_len));
@@ -2505,7 +2500,8 @@ __device__ __forceinline__ void attn_rows_softmax(float* __restrict__ sc, uint32
     }
 }
 
-template <int G, int HS, int NWAVES>
+// TABLE: the blocks of rows from a table (attn_blocks), else every R rows
+template <int G, int HS, int NWAVES, bool TABLE>
 __global__ __launch_bounds__(64 * NWAVES) void k_attn_rows(const float* __restrict__ q, float* __restrict__ out,
                                                    float* __restrict__ att, const float* __restrict__ kc,
                                                    const float* __restrict__ vc, size_t loff,
@@ -2528,8 +2524,8 @@ __global__ __launch_bounds__(64 * NWAVES) void k_attn_rows(const float* __restri
     // the last row blocks first: a causal prefill's windows grow with the
     // row, so the longest blocks start first and the short ones fill in behind
     const uint32_t bi = gridDim.y - 1 - blockIdx.y;
-    const uint32_t r0 = blocks ? blocks[bi] : bi * R;
-    const uint32_t nr = blocks ? blocks[bi + 1] - r0 : min(R, n_rows - r0);
+    const uint32_t r0 = TABLE ? blocks[bi] : bi * R;
+    const uint32_t nr = TABLE ? blocks[bi + 1] - r0 : min(R, n_rows - r0);
     // query heads h0 .. h0 + G - 1 of KV head h0 / kv_mul (G divides kv_mul)
     const uint32_t width = n_heads * HS, h0 = blockIdx.x * G, kvo = (h0 / kv_mul) * HS;
     const DevWindow w0 = windows[r0];
@@ -3029,8 +3025,7 @@ hipError_t launch_attention_split_rows(hipStream_t st, const float* q, float* ou
         return hipErrorInvalidValue;
     const size_t n_kv = n_heads / kv_mul, nchunks = (max_count + 63) / 64, loff = layer * seq_len * kv_dim;
     const size_t scs = (max_count + 3) & ~(size_t)3;
-    const size_t cap = attention_split_cap(max_count, seq_len);  // the scratch's row stride
-    const uint32_t ss = (uint32_t)((cap + 3) & ~(size_t)3), ms = (uint32_t)attn_split_ms(cap);
+    const uint32_t ss = (uint32_t)((seq_len + 3) & ~(size_t)3), ms = (uint32_t)attn_split_ms(seq_len);
     float* sc = scratch;
     float* mxp = scratch + n_rows * n_heads * ss;
     const size_t lds = (kv_mul * scs + 64 * hs) * sizeof(float);
@@ -3099,49 +3094,98 @@ static std::vector<uint32_t> attn_blocks(const DevWindow* w, size_t n_rows, size
     return b;
 }
 
-// Which launches take `n_rows` rows with the given windows. Rows whose blocks
-// share a window layout (a prefill, also of several sequences, whose blocks the
-// table keeps apart) can run by blocks: on the matrix core (attn_mx.hip) for
-// long windows, else k_attn_rows. Both are as long as their longest block
-// however few there are, so up to some number of (row, KV head) pairs the
-// per-row launches are shorter. us, blocks / per row: 15/5 heads of 64, 9 rows
-// at 512 36 / 18, 128 rows at 512 42.9 / 41.4, 32 rows at 2000 224 / 74, 200
-// rows at 900 133 / 94; 32/32 heads of 64, 16 rows at 200 19.0 / 16.9, 64 rows
-// 22 / 36; 64 rows at 900 120 / 136; 16/8 heads of 128, 32 rows at 0 18.9 / 9.3,
-// 200 rows at 100 53 / 42, 250 rows at 0 44 / 43, 128 rows at 1500 214 / 149.
-// Sequences of their own lengths, blocks by the table: 24 of 700 rows in all,
-// 15/5 heads 19.9 / 30.8, 16/8 heads of 128 108 / 62; 8 of 1500 rows 89 / 247.
+// The per-row launches against blocks of rows. Blocks (k_attn_rows, attn_mx.hip)
+// read a window's keys and values once for all their rows, but a launch is as long as
+// its longest block however few there are; per row, every row reads its own. So
+// per row is shorter up to some number of (row, KV head) pairs, fewer where a
+// block's matrix work serves more query heads, more where short windows leave a
+// block little to share. The lines lie where the blocks overtake over one
+// sequence's rows (2 to 320 of them at windows from 1 to 4020, 26 shapes of heads
+// of 32, 64 and 128); past them per row costs up to twice as much. us, per row / blocks:
+//   matrix core  32/8 heads of 128, 128 rows at 1000 161 / 157, 200 rows at 3000 827 / 393
+//                16/8 heads of 128, 128 rows at 1500 159 / 214, 200 rows at 3000 529 / 392
+//                12/4 heads of 128, 160 rows at 300 62 / 74, 320 rows at 3000 625 / 406
+//                15/5 heads of 64, 200 rows at 1000 108 / 142, 256 rows at 3000 406 / 350
+//   k_attn_rows  15/5 heads of 64, 12 rows at 60 13.8 / 11.8, 12 rows at 400 17.6 / 30.0
+//                16/2 heads of 64, 32 rows at 60 22.7 / 12.2, 24 rows at 600 41.3 / 41.8
+//                32/32 heads of 64, 12 rows at 130 15.7 / 14.5
 // Heads of 128 below the matrix-core windows: a wave of k_attn_rows scores 64
 // positions for all of its block's pairs, so windows this short leave most of
-// its waves idle there, and per row is shorter at any number of rows of several
-// query heads per KV head (sequences of 40-90, 16/8 heads: 250 rows 41 / 30, 2000 rows
-// 346 / 181; 32/8 heads 77 / 39, 677 / 260), and of one up to some 2000 pairs
-// (8/8 heads: 100 rows 21 / 19, 250 rows 37 / 35, 500 rows 55 / 60, 2000 rows
-// 175 / 210).
+// its waves idle there, and per row is shorter at any number of rows of two to
+// four query heads per KV head (16/8 heads, sequences of 40-90: 250 rows 30 / 41,
+// 2000 rows 181 / 346), of one up to some 2000 pairs (8/8 heads, 500 rows 60 / 55).
+static size_t attn_mx_pairs(size_t max_count, size_t kv_mul, size_t hs) {
+    const size_t lim = kv_mul == 8 ? 512 : hs == 64 ? 1280 : kv_mul == 3 ? 640 : 1024;
+    return max_count > 1536 ? lim * 3 / 4 : lim;
+}
+static size_t attn_rows_pairs(size_t max_count, size_t kv_mul, size_t hs) {
+    if (hs == 128) return kv_mul == 1 ? 2048 : kv_mul < 8 ? SIZE_MAX : 0;
+    if (max_count <= 64 * kv_mul) return 0;
+    return kv_mul == 8 ? 256 : kv_mul == 1 && hs == 64 && max_count < 200 ? 320 : 512;
+}
+
+// Which launches take `n_rows` rows with the given windows. Rows whose blocks
+// share a window layout (a prefill) can run by blocks: on the matrix core for long
+// windows, else on k_attn_rows; sequences that end inside a block have a table
+// keep theirs apart. Such blocks are less full and one for each sequence at least, so
+// they need twice the pairs on the matrix core, windows below its range on
+// k_attn_rows, and heads of 64 there: 24 sequences of 700 rows in all, 15/5 heads of
+// 64 31 us per row / 20 by blocks; 8 of 1500 rows, heads of 128 247 / 89; but
+// 700 rows of sequences of 2-6 behind 1200 shared positions 294 / 678 on
+// k_attn_rows, 100 of 40-90, 16/8 heads of 32 11.5 / 17. Groupings without per-row
+// launches, a workgroup per row / by blocks: sequences of 8-24, 12/2 heads of 64 behind
+// 1200 positions 100 rows 76 / 142, 700 rows 614 / 194; 12/2 heads of 128 behind 150,
+// 100 rows 23 / 40, 400 rows 124 / 43.
 AttnPlan attention_plan(const DevWindow* w, size_t n_rows, size_t max_count, size_t n_heads, size_t kv_mul,
                         size_t hs, bool per_row, bool tables) {
     AttnPlan p;
     const size_t pairs = n_rows * (n_heads / kv_mul);
     const bool split = attention_split_rows_ok(max_count, kv_mul, hs);
     const bool choice = split && per_row && n_rows <= 65535;  // a grid dimension counts the rows
-    if (n_rows < 2) {  // k_attention_fast up to 256 positions of small heads (9 against 9.5 us)
-        if (choice && (max_count >= 256 || hs == 128)) p.kind = ATTN_SPLIT;
+    if (n_rows < 2) {
+        // k_attention_fast for short windows (us, per row / fast: 15/5 heads of 64 at 160 9.6 / 8.1, at 300 10.4 /
+        // 11.0, 32/16 heads of 128 at 160 13.1 / 11.8) and where eight score rows leave little LDS (16/2 heads of 32
+        // at 3700 131 / 111)
+        const bool little = kv_mul == 8 && hs < 128 && max_count > 3072;
+        if (choice && max_count >= (hs == 32 ? 512 : 256) && !little) p.kind = ATTN_SPLIT;
         return p;
     }
-    auto blocked = [&](size_t R) {  // blocks at least half full, or the regular ones
-        p.blocks = attn_blocks(w, n_rows, R);
-        return p.blocks.empty() || (tables && R > 1 && (p.blocks.size() - 1) * R <= 2 * n_rows);
-    };
+    const size_t mx = attention_mx_rows(max_count, kv_mul, hs);
     const size_t nw = attn_rows_waves(attn_rows_group(kv_mul), hs, max_count);
-    if (attention_mx_rows(max_count, kv_mul, hs) && blocked(attention_mx_rows(max_count, kv_mul, hs))) {
-        p.kind = choice && pairs <= (hs == 128 ? 1792 : 1280) ? ATTN_SPLIT : ATTN_MX;
-    } else if (nw && blocked(nw * (128 / hs) / attn_rows_group(kv_mul))) {
-        const bool shorter = hs == 128 ? kv_mul > 1 || pairs <= 2048 : max_count > 64 && pairs <= 512;
-        p.kind = choice && shorter ? ATTN_SPLIT : ATTN_ROWS;
-    } else {
-        p.kind = split ? ATTN_SPLIT : ATTN_GENERAL;
+    const size_t rows = nw ? nw * (128 / hs) / attn_rows_group(kv_mul) : 0;
+    // a table's blocks at least half full; where no per-row launches apply, enough work against k_attention_fast
+    const bool many = n_rows * n_heads >= (hs == 128 ? 4096 : 8192);
+    auto irregular_ok = [&](size_t R) { return tables && R > 1 && (p.blocks.size() - 1) * R <= 2 * n_rows; };
+    if (mx) {
+        const size_t lim = attn_mx_pairs(max_count, kv_mul, hs);
+        p.blocks = attn_blocks(w, n_rows, mx);
+        if (p.blocks.empty()) {
+            p.kind = choice && pairs <= lim ? ATTN_SPLIT : ATTN_MX;
+            return p;
+        }
+        if (irregular_ok(mx) && (split ? pairs > 2 * lim : many)) {
+            p.kind = ATTN_MX;
+            return p;
+        }
     }
-    if (p.kind == ATTN_SPLIT || p.kind == ATTN_GENERAL) p.blocks.clear();
+    if (rows) {
+        // at matrix-core windows k_attn_rows has small blocks, down to a row each (us, per row / by its blocks: 100 rows
+        // of 12/4 heads of 128 at 1224 103 / 83; 200 rows of 16/2 heads of 128, a row a block, at 156 35 / 52)
+        const size_t lim = !mx         ? attn_rows_pairs(max_count, kv_mul, hs)
+                           : rows == 1 ? SIZE_MAX
+                                       : attn_mx_pairs(max_count, kv_mul, hs) / 2;
+        p.blocks = attn_blocks(w, n_rows, rows);
+        if (p.blocks.empty()) {
+            p.kind = choice && pairs <= lim ? ATTN_SPLIT : ATTN_ROWS;
+            return p;
+        }
+        if (hs == 64 && irregular_ok(rows) && (split ? !mx && pairs > std::max<size_t>(256, lim) : many)) {
+            p.kind = ATTN_ROWS;
+            return p;
+        }
+    }
+    p.kind = split ? ATTN_SPLIT : ATTN_GENERAL;
+    p.blocks.clear();
     return p;
 }
 
@@ -3197,28 +3241,31 @@ hipError_t launch_attention(hipStream_t st, const float* q, float* out, float* a
                                    kv_dim, seq_len, scale, qo, so, ho, mx_scratch, keep_att, blocks, n_blocks);
     }
     if (plan.kind == ATTN_ROWS) {
-        // many rows whose blocks share a window layout: k_attn_rows
+        // many rows whose blocks share a window layout: k_attn_rows, tables for heads of 64 alone (attention_plan)
+        if (blocks && hs != 64) return hipErrorInvalidValue;
         const size_t G = attn_rows_group(kv_mul), nw = attn_rows_waves(G, hs, max_count);
         const size_t R = (nw * (128 / hs)) / G;  // rows per block: AttnRowsShape
         const size_t lds = attn_rows_lds(G, hs, max_count, nw);
         const uint32_t scs = (uint32_t)((max_count + 3) & ~(size_t)3);
         const dim3 grid((unsigned)(n_heads / G), (unsigned)(blocks ? n_blocks : (n_rows + R - 1) / R));
-#define KR_ATTN_ROWS(g, h, w)                                                                                 \
-    hipLaunchKernelGGL((k_attn_rows<g, h, w>), grid, dim3(64 * w), lds, st, q, out, keep_att ? att : nullptr, kc,   \
+#define KR_ATTN_ROWS(g, h, w, t)                                                                              \
+    hipLaunchKernelGGL((k_attn_rows<g, h, w, t>), grid, dim3(64 * w), lds, st, q, out, keep_att ? att : nullptr, kc, \
                        vc, layer * seq_len * kv_dim, windows, (uint32_t)n_rows, (uint32_t)n_heads,              \
                        (uint32_t)kv_mul, (uint32_t)kv_dim, (uint32_t)seq_len, scale, scs, qo, so, ho, blocks)
-#define KR_ATTN_ROWS_W(g, h)         \
+#define KR_ATTN_ROWS_W(g, h, t)      \
     if (nw == 8)                     \
-        KR_ATTN_ROWS(g, h, 8);       \
+        KR_ATTN_ROWS(g, h, 8, t);    \
     else                             \
-        KR_ATTN_ROWS(g, h, 4);
-#define KR_ATTN_ROWS_G(g)          \
-    if (hs == 32)                  \
-        KR_ATTN_ROWS_W(g, 32)      \
-    else if (hs == 64)             \
-        KR_ATTN_ROWS_W(g, 64)      \
-    else                           \
-        KR_ATTN_ROWS_W(g, 128)
+        KR_ATTN_ROWS(g, h, 4, t);
+#define KR_ATTN_ROWS_G(g)            \
+    if (hs == 32)                    \
+        KR_ATTN_ROWS_W(g, 32, false) \
+    else if (hs == 128)              \
+        KR_ATTN_ROWS_W(g, 128, false) \
+    else if (blocks)                 \
+        KR_ATTN_ROWS_W(g, 64, true)  \
+    else                             \
+        KR_ATTN_ROWS_W(g, 64, false)
         switch (G) {
             case 8: KR_ATTN_ROWS_G(8) break;
             case 4: KR_ATTN_ROWS_G(4) break;

@@ -66,10 +66,13 @@ def test_a_capture_takes_no_table_and_no_new_scratch_for_regular_rows(geometry):
 
 
 def test_large_scratch_is_not_taken_by_choice():
-    # 200 rows of 16 heads: 12.8 MB of scores at 1024 slots, 1.6 GB at 131072
-    ws = [Window(0, 100 + i) for i in range(200)]
+    # 100 rows of 16 heads: 6.6 MB of scores at 1024 slots, 0.84 GB at 131072
+    ws = [Window(0, 100 + i) for i in range(100)]
     assert attention_plan(ws, spec(16, 8, 128, 1024))[0] == "split"
-    assert attention_plan(ws, spec(16, 8, 128, 131072))[0] != "split"
+    assert attention_plan(ws, spec(16, 8, 128, 131072))[0] == "mx"
+    # rows without blocks have nothing else
+    ws = [Window(50 * i, 50 * i + 20) for i in range(100)]
+    assert attention_plan(ws, spec(16, 8, 128, 131072))[0] == "split"
 
 
 def test_short_windows_of_128_wide_heads():
@@ -82,6 +85,45 @@ def test_short_windows_of_128_wide_heads():
     assert attention_plan(equal(2000, 40), spec(16, 8, 128, 2048))[0] == "split"
     # more rows than a grid dimension has workgroups
     assert attention_plan([Window(0, 0)] * 65536, spec(2, 1, 128, 8))[0] == "rows"
+
+
+# both sides of the lines at which blocks overtake the per-row launches: rows of
+# one sequence ending at `end`
+@pytest.mark.parametrize("geometry,n,end,kind", [
+    ((16, 8, 128), 128, 1536, "split"), ((16, 8, 128), 129, 1536, "mx"), ((16, 8, 128), 96, 1537, "split"),
+    ((16, 8, 128), 97, 1537, "mx"), ((12, 4, 128), 160, 500, "split"), ((12, 4, 128), 161, 500, "mx"),
+    ((16, 2, 128), 256, 900, "split"), ((16, 2, 128), 257, 900, "mx"), ((16, 4, 64), 320, 1000, "split"),
+    ((16, 4, 64), 321, 1000, "mx"), ((15, 5, 64), 192, 3000, "split"), ((15, 5, 64), 193, 3000, "mx"),
+    ((15, 5, 64), 100, 193, "split"), ((15, 5, 64), 100, 192, "rows"), ((15, 5, 64), 103, 400, "rows"),
+    ((16, 16, 64), 20, 199, "split"), ((16, 16, 64), 21, 199, "rows"), ((16, 16, 64), 32, 200, "split"),
+    ((16, 2, 64), 100, 513, "split"), ((16, 2, 64), 100, 512, "rows"), ((16, 2, 64), 129, 600, "rows"),
+    ((8, 1, 128), 20, 100, "rows"), ((32, 8, 128), 140, 150, "split"), ((16, 2, 32), 64, 100, "rows"),
+    ((15, 5, 64), 1, 255, "general"), ((15, 5, 64), 1, 256, "split"), ((16, 8, 128), 1, 255, "general"),
+    ((16, 2, 32), 1, 511, "general"), ((16, 2, 32), 1, 3072, "split"), ((16, 2, 32), 1, 3073, "general"),
+    ((16, 2, 64), 1, 3073, "general"), ((16, 2, 128), 1, 3073, "split"),
+])
+def test_lines_between_rows_and_blocks(geometry, n, end, kind):
+    ws = [Window(0, end - n + i) for i in range(n)]
+    assert attention_plan(ws, spec(*geometry, 4096)) == (kind, [])
+
+
+# sequences of their own lengths: tables where they are shorter than the per-row launches
+@pytest.mark.parametrize("geometry,lens,shared,kind", [
+    ((15, 5, 64), [10, 11, 9, 13, 7], 0, "split"), ((15, 5, 64), [50, 51, 52, 53, 7], 0, "rows"),
+    ((16, 8, 32), [50, 51, 52, 53, 57] * 3, 0, "split"), ((16, 8, 128), [50, 51, 52, 53, 7], 0, "split"),
+    ((15, 5, 64), [3, 4, 5, 2] * 50, 1200, "split"), ((15, 5, 64), [103, 104, 105, 201], 1200, "mx"),
+    ((16, 8, 128), [103, 104, 105], 200, "mx"), ((16, 8, 128), [83, 84, 85], 200, "split"),
+    ((12, 2, 128), [101, 102, 103, 50], 150, "mx"), ((12, 2, 128), [101, 102, 103], 150, "general"),
+    ((12, 2, 64), [101, 102, 103] * 3, 0, "rows"), ((12, 2, 64), [101, 102, 103] * 2, 0, "general"),
+    ((12, 1, 32), [101, 102, 103] * 9, 0, "general"),
+])
+def test_lines_for_ragged_sequences(geometry, lens, shared, kind):
+    ws, base = [], shared
+    for n in lens:
+        ws += [Window(base, base + i, (0, shared)) for i in range(n)]
+        base += n
+    got, blocks = attention_plan(ws, spec(*geometry, 4096))
+    assert got == kind and bool(blocks) == (kind in ("rows", "mx"))
 
 
 def test_refused_windows():

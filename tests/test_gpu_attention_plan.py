@@ -28,11 +28,13 @@ def ragged(lens, shared=0):
 # one row: below and at the split's first window, 4- and 16-dim slices (n_kv hs
 # / 4 workgroups up to and past 256), passes of the V slice
 @pytest.mark.parametrize("n_heads,n_kv,hs,count", [
-    (15, 5, 64, 255), (15, 5, 64, 256), (32, 32, 64, 700), (16, 8, 128, 3), (32, 16, 128, 2900), (4, 2, 32, 300),
+    (15, 5, 64, 255), (15, 5, 64, 256), (32, 32, 64, 700), (16, 8, 128, 3), (16, 8, 128, 300), (32, 16, 128, 2900),
+    (4, 2, 32, 300), (4, 2, 32, 512), (16, 2, 64, 3072), (16, 2, 64, 3073),
 ])
 def test_one_row(n_heads, n_kv, hs, count):
     kinds = _attention_case(count + 5, n_heads, n_kv, hs, [(2, count + 1, 0, 0)], count)
-    assert kinds == (["general"] if count == 255 else ["split", "general"])
+    general = count < (512 if hs == 32 else 256) or count == 3073
+    assert kinds == (["general"] if general else ["split", "general"])
 
 
 # few rows at long windows: slices of 4 and 16 dims, a workgroup per (row, KV
@@ -55,16 +57,17 @@ def test_rows_of_one_sequence(n_heads, n_kv, hs, n, start):
     (15, 5, 64, [1, 5, 6, 37, 64, 3, 2, 1], 0, "rows"), (15, 5, 64, [70, 33, 48], 9, "rows"),
     (4, 4, 64, [7, 50, 1, 9], 20, "split"), (6, 2, 64, [1, 1, 2, 1, 1], 0, "split"),
     (16, 8, 128, [100, 30, 66, 1], 0, "split"), (16, 8, 128, [180, 17, 1, 15], 12, "split"),
-    (16, 8, 128, [180, 17, 1, 30], 12, "mx"), (4, 2, 64, [790, 30, 1], 0, "mx"), (8, 4, 32, [40, 3, 25], 7, "rows"),
-    (8, 8, 128, [90, 60, 40, 30, 44], 0, "rows"), (12, 2, 128, [31, 50, 3], 5, "rows"),
-    (4, 4, 64, [790, 30, 1], 9, "mx"), (16, 4, 128, [300, 120, 60], 4, "mx"), (16, 2, 64, [790, 30, 1], 0, "mx"),
+    (16, 8, 128, [180, 17, 1, 70], 12, "mx"), (4, 2, 64, [790, 495, 1], 0, "mx"), (8, 4, 32, [40, 3, 25], 7, "split"),
+    (12, 1, 32, [40, 3, 25], 7, "general"), (8, 8, 128, [90, 60, 40, 30, 44], 0, "split"),
+    (12, 2, 64, [99, 101, 98, 97, 103, 102, 95], 3, "rows"), (12, 2, 128, [190, 150, 3], 5, "mx"), (4, 4, 64, [790, 30, 1], 9, "mx"), (16, 4, 128, [300, 120, 100], 4, "mx"),
+    (16, 2, 64, [790, 30, 1], 0, "mx"),
 ])
 def test_rows_of_ragged_sequences(n_heads, n_kv, hs, lens, shared, kind):
     wins = ragged(lens, shared)
     kinds = _attention_case(shared + sum(lens) + 2, n_heads, n_kv, hs, wins, sum(lens) + shared)
     spec = K.AttnSpec(n_heads, n_heads // n_kv, hs, n_kv * hs, shared + sum(lens) + 2)
     _, blocks = K.backends.attention_plan([K.Window(a, s, (x, y)) for a, s, x, y in wins], spec)
-    assert kinds[0] == kind and bool(blocks) == (kind != "split")
+    assert kinds[0] == kind and bool(blocks) == (kind in ("rows", "mx"))
 
 
 @pytest.mark.parametrize("n,hs", [(1, 64), (1, 128), (6, 64)])
