@@ -2174,6 +2174,18 @@ static size_t attn_slice_dims(size_t blocks, size_t max_count, size_t G, size_t 
     return 0;
 }
 
+// The same for launch_attention_split_rows, `quant` where the slices leave the Q8
+// blocks to a launch of their own. Several rows of short windows have little
+// softmax to spread, and eight query heads a slice of 16 dims too little of the
+// LDS: a workgroup per pair then. us, 4 / 16 / pair: 32 rows at 4 of 16/2 heads of 32
+// 19 / 20 / 9.7, 12 rows at 12 of 15/5 heads of 64 20 / 13.3 / 8.9, 6 at 211 of 16/8
+// heads of 64 16 / 13.5 / 13.1, 16 at 1981 of 16/2 heads of 64 68 / 106 / 70.
+static size_t attn_row_slices(size_t n_rows, size_t n_kv, size_t max_count, size_t G, size_t hs, bool quant) {
+    const size_t dw = attn_slice_dims(n_rows * n_kv, max_count, G, hs);
+    const bool pair = max_count < 64 * G + (quant ? 192 : 64) || (dw == 16 && G == 8);
+    return n_rows > 1 && pair ? 0 : dw;
+}
+
 bool attention_split_ok(size_t max_count, size_t kv_mul, size_t hs) {
     if (kv_mul != 1 && kv_mul != 2 && kv_mul != 3 && kv_mul != 4 && kv_mul != 8) return false;
     if (hs != 32 && hs != 64 && hs != 128) return false;
@@ -3030,7 +3042,8 @@ hipError_t launch_attention_split_rows(hipStream_t st, const float* q, float* ou
     float* mxp = scratch + n_rows * n_heads * ss;
     const size_t lds = (kv_mul * scs + 64 * hs) * sizeof(float);
     const dim3 g1((unsigned)n_kv, (unsigned)nchunks, (unsigned)n_rows), g2((unsigned)n_kv, (unsigned)n_rows);
-    const size_t dw = attn_slice_dims(n_rows * n_kv, max_count, kv_mul, hs), dws = dw ? dw : kAttnSplitDW;
+    const size_t dw = attn_row_slices(n_rows, n_kv, max_count, kv_mul, hs, qo != nullptr);
+    const size_t dws = dw ? dw : kAttnSplitDW;
     const size_t pw = attn_split_pass(scs, kv_mul, dws), lds3 = attn_split_lds(scs, kv_mul, dws, pw);
     const dim3 g3((unsigned)(n_kv * (hs / dws)), (unsigned)n_rows);
     if (!keep_att) att = nullptr;

@@ -70,6 +70,17 @@ def test_rows_of_ragged_sequences(n_heads, n_kv, hs, lens, shared, kind):
     assert kinds[0] == kind and bool(blocks) == (kind in ("rows", "mx"))
 
 
+# a batch of sequences: a workgroup per (row, KV head), slices of 4 and of 16 dims,
+# on both sides of their shortest window; eight query heads without slices of 16
+@pytest.mark.parametrize("n_heads,n_kv,hs,n,count", [
+    (15, 5, 64, 2, 255), (15, 5, 64, 2, 256), (15, 5, 64, 6, 256), (15, 5, 64, 13, 256), (8, 8, 128, 2, 127),
+    (8, 8, 128, 2, 128), (16, 2, 64, 8, 576), (16, 2, 64, 9, 576), (16, 8, 32, 3, 200), (8, 4, 32, 32, 200),
+])
+def test_independent_rows(n_heads, n_kv, hs, n, count):
+    windows = [(count * i, count * i + count - 1 - 3 * (i % 4), 0, 0) for i in range(n)]
+    assert "split" in _attention_case(count * n + 1, n_heads, n_kv, hs, windows, n + count)
+
+
 @pytest.mark.parametrize("n,hs", [(1, 64), (1, 128), (6, 64)])
 def test_growing_windows_leave_the_scratch_in_place(n, hs):
     # a conversation's window grows past 512, 1024, 1536 positions: what the
