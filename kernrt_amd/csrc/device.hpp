@@ -178,8 +178,8 @@ hipError_t launch_direct_swi(hipStream_t st, int sem, const MatSet& ms, size_t k
 hipError_t launch_direct_rope(hipStream_t st, int sem, const MatSet& ms, size_t k, QuantAct x, size_t rows,
                               RopeOut ro);
 // The Q8_0x4 forms by grid: direct up to kDirectTiles16 16x16 units (one wave
-// each), then 64x64 tiles (a 32x32 unit per wave) up to kChainTiles64 of them,
-// then 128x128 tiles (32x64 per wave). The two forms with an epilogue count
+// each), then 64x64 tiles (a 32x32 unit per wave) or 128x128 (32x64 per wave) by
+// the rounds of them (gemm.hip). The two forms with an epilogue count
 // workgroups of four 16x16 units. us, direct / 64x64 tiles, Q8_0x4:
 //   SiLU  2560x960: 240 workgroups 8.7 / 12.4, 320 10.5 / 13.0, 480 10.7 / 13.1, 560 13.9 / 13.1
 //         4608x1536: 144 8.7 / 15.1, 432 13.2 / 15.7, 576 17.3 / 16.4; 8192x2048: 256 11 / 18, 512 16 / 17, 768 21 / 18
@@ -187,7 +187,7 @@ hipError_t launch_direct_rope(hipStream_t st, int sem, const MatSet& ms, size_t 
 //         6144x2048: 192 10.0 / 15.8, 384 14.3 / 18.4, 480 14.5 / 18.4, 576 19.7 / 18.2
 // Both cross near two workgroups per CU (512). The RoPE line lies below that at
 // 400, the SiLU line at one per CU, where direct is well ahead.
-static constexpr size_t kDirectTiles16 = 1408, kChainTiles64 = 640, kDirectSwiMax = 256, kDirectRopeMax = 400;
+static constexpr size_t kDirectTiles16 = 1408, kDirectSwiMax = 256, kDirectRopeMax = 400;
 
 // The chunk pipeline of k_gemm_q8_s16 (gemm.hip). At chunk c, the register
 // stage (c + 1) % NS holds chunk c + 1 and LDS buffer c & 1 holds chunk c.

@@ -762,11 +762,18 @@ static hipError_t gemm_q8_go(hipStream_t st, const MatSet& ms, size_t k, QuantAc
 //   960x2560   77 rows  7.7 / 16.0 / 36 (23.2)   700 rows 23.1 / 16.7 / 36 (23.6)
 //   9216x1536  32 rows 10.8 / 12.0 / 23 (17.0)   128 rows 25.2 / 18.2 / 25 (23.3)
 //   5120x960  700 rows 38.6 / 23.6 / 19 (29.4)  16384x2048, 256 rows 97 / 44 / 37 (59)
-// Direct wins to about 1400 16x16 units, 128x128 from about 640 64x64 tiles.
+// Direct wins to about 1400 16x16 units. Beyond, a launch is as long as its rounds
+// of one tile per CU, and a round of 128x128 tiles takes a little over three of
+// 64x64 (3072 wide: 12.2 us a round of 64x64, 38 of 128x128; a second round of
+// 64x64 shares the CUs with the first): 9216x3072, 400 rows 49.6 in 4 rounds / 76.8
+// in 2, 256 rows 40.8 in 3 / 39.7 in 1; 12288x960, 300 rows 22.1 / 31.8.
+static bool chain_tiles64(size_t tiles64, size_t tiles128) {
+    return tiles64 <= 512 || (tiles64 + 255) / 256 < 3 * ((tiles128 + 255) / 256);
+}
 static hipError_t gemm_chain_go(hipStream_t st, const MatSet& ms, size_t k, QuantAct x, size_t rows, int32_t* dbg) {
     if ((rows + 15) / 16 * gemm_col_tiles(ms, 16) <= kDirectTiles16)
         return launch_gemm_direct(st, SEM_FMA_CHAIN, ms, k, x, rows, dbg);
-    if ((rows + 63) / 64 * gemm_col_tiles(ms, 64) <= kChainTiles64)
+    if (chain_tiles64((rows + 63) / 64 * gemm_col_tiles(ms, 64), (rows + 127) / 128 * gemm_col_tiles(ms, 128)))
         launch_q8<SEM_FMA_CHAIN, 64, 64, 1, 4, 4, 3, 2, 2>(st, ms, x, rows, k, dbg);
     else
         launch_q8<SEM_FMA_CHAIN, 128, 128, 2, 4, 4, 2, 1, 1>(st, ms, x, rows, k, dbg);
@@ -802,7 +809,7 @@ hipError_t launch_qkv_rope(hipStream_t st, const DevMatrix& q, const DevMatrix& 
     const RopeOut ro{pos, slots, tab, kc, vc, (uint32_t)k.n};
     if (q.storage == KR_STORAGE_Q8_0X4) {
         if (qkv_rope_direct(q, k, rows)) return launch_direct_rope(st, SEM_FMA_CHAIN, ms, q.k, x, rows, ro);
-        if ((rows + 63) / 64 * ((q.n + 2 * k.n) / 64) <= kChainTiles64)
+        if (chain_tiles64((rows + 63) / 64 * gemm_col_tiles(ms, 64), (rows + 127) / 128 * gemm_col_tiles(ms, 128)))
             launch_q8_rope<SEM_FMA_CHAIN, 64, 64, 1, 4, 4, 3, 2, 2>(st, ms, x, rows, q.k, ro);
         else
             launch_q8_rope<SEM_FMA_CHAIN, 128, 128, 2, 4, 4, 2, 1, 1>(st, ms, x, rows, q.k, ro);
@@ -849,7 +856,7 @@ hipError_t launch_gate_up_silu(hipStream_t st, const DevMatrix& gate, const DevM
     const size_t m128 = (rows + 127) / 128, blocks = gate.n / 32, direct = (rows + 15) / 16 * blocks;
     if (gate.storage == KR_STORAGE_Q8_0X4) {
         if (direct <= kDirectSwiMax) return launch_direct_swi(st, SEM_FMA_CHAIN, ms, gate.k, x, rows, so);
-        if ((rows + 63) / 64 * blocks <= kChainTiles64)
+        if (chain_tiles64((rows + 63) / 64 * blocks, m128 * ((blocks + 1) / 2)))
             launch_q8_swi<SEM_FMA_CHAIN, 64, 64, 1, 4, 4, 3, 2, 2>(st, ms, x, rows, gate.k, so);
         else
             launch_q8_swi<SEM_FMA_CHAIN, 128, 128, 2, 4, 4, 2, 1, 1>(st, ms, x, rows, gate.k, so);
