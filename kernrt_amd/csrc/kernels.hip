@@ -1169,17 +1169,20 @@ bool swiglu_fusable(const DevMatrix& gate, const DevMatrix& up) {
 // From how many rows on a projection takes the matrix core (gemm.hip). The GEMV
 // serves four rows per pass over the weights, so five to seven rows cost two
 // passes: 960x2560 Q8_0x4, 6 rows, 9.1 against 7.3 us direct; 5120x960 9.7
-// against 5.2. With the four partial sums the direct form needs a wide output to
-// win (4096x1024 7.9 against 5.5 us, but 1024x2048 6.2 against 6.9).
-static size_t gemm_min_rows(int sem, const MatSet& ms) {
+// against 5.2. The direct form is as long as one chain over the inner dimension k,
+// so a narrow output of long rows stays with the GEMV (Q8_0x4, 5 rows: 64x8192 9.1
+// against 16.1, 576x8192 13.0 / 16.3, 576x4608 11.0 / 10.4); with the four partial
+// sums it needs a wide output to win (4096x1024 7.9 against 5.5 us, but 1024x2048
+// 6.2 against 6.9).
+static size_t gemm_min_rows(int sem, const MatSet& ms, size_t k) {
     size_t n = 0;
     for (int i = 0; i < ms.count; i++) n += ms.n[i];
-    return sem == SEM_FMA_CHAIN || n >= 3200 ? 5 : 8;
+    return n >= (sem == SEM_FMA_CHAIN ? k / 8 : 3200) ? 5 : 8;
 }
 
 template <int SEM>
 static hipError_t gemv_rows(hipStream_t st, const MatSet& ms, size_t k, QuantAct x, size_t rows, int32_t* dbg) {
-    if (rows >= gemm_min_rows(SEM, ms)) return launch_gemm_q8(st, SEM, ms, k, x, rows, dbg);
+    if (rows >= gemm_min_rows(SEM, ms, k)) return launch_gemm_q8(st, SEM, ms, k, x, rows, dbg);
     size_t nb = k / 32;
     size_t done = 0;
     while (done < rows) {

@@ -41,11 +41,12 @@ def test_direct_gemm_edges(hip, storage, k, rows, n):
 
 # both sides of the dispatch: 1408 units of 16x16 (64x64 tiles above), 512 tiles
 # of 64x64 (128x128 above, 64x64 again where those take a second round) for
-# Q8_0x4; 512 units for Q8_0
+# Q8_0x4; 512 units for Q8_0; five to seven rows of a narrow output (GEMV below
+# an eighth of the inner dimension)
 @pytest.mark.parametrize("storage,n,k,rows", [
     ("q8_0x4", 4096, 160, 80), ("q8_0x4", 4096, 160, 96), ("q8_0x4", 4100, 96, 130),
     ("q8_0x4", 4096, 96, 512), ("q8_0x4", 4096, 96, 513), ("q8_0x4", 4096, 96, 640), ("q8_0x4", 4164, 160, 700),
-    ("q8_0x4", 9216, 96, 385), ("q8_0", 2048, 96, 64), ("q8_0", 2048, 96, 80),
+    ("q8_0x4", 9216, 96, 385), ("q8_0x4", 64, 544, 5), ("q8_0x4", 68, 544, 7), ("q8_0", 2048, 96, 64), ("q8_0", 2048, 96, 80),
 ])
 def test_gemm_dispatch_edges(hip, storage, n, k, rows):
     check_matmul(hip, storage, n, k, rows)
