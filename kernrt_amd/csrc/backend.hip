@@ -648,6 +648,12 @@ kr::QuantAct act(kr_ctx* c) { return kr::QuantAct{c->wq, c->ws, c->wh}; }
 // the matrices. A single row of up to 2048 is quantized inside that launch, by
 // every workgroup for itself (960 wide, q/k/v: one launch of 4.0 us for four of
 // 2.7 + 3.8 + 3.6 + 3.6); a wider row takes longer to quantize again than to launch.
+// So does a set with very many outputs, since its workgroups grow with it. Both
+// forms, Q8_0x4, us (in the launch / before it), by k x outputs in all:
+//   2048 x 8192: 7.8 / 8.0   2048 x 12288: 9.9 / 9.3    2048 x 16384: 11.9 / 10.6
+//   1536 x 18432: 10.2 / 10.3   1536 x 24576: 12.4 / 11.7   1536 x 49152: 20.9 / 17.5
+//   960 x 49152: 11.8 / 12.9    960 x 98304: 20.9 / 20.0
+// They cross where k * k * outputs is 3 << 34 (at 960, half as far again).
 // Outputs that repeat or are x keep the order of separate launches.
 int project_many(kr_ctx* c, size_t layer, const int* projs, const kr_buf* ys, int n, kr_buf x, size_t rows) {
     CHECK(c, c->prepared, "prepare() runs before any compute");
@@ -665,14 +671,16 @@ int project_many(kr_ctx* c, size_t layer, const int* projs, const kr_buf* ys, in
     size_t k = ms[0]->m.k;
     BUF(xb, x, rows * k);
     bool one = true, apart = true;
+    size_t outs = 0;
     for (int i = 0; i < n; i++) {
         BUF(yb, ys[i], rows * ms[i]->m.n);
         yp[i] = yb->p;
+        outs += ms[i]->m.n;
         one = one && ws[i]->storage == ws[0]->storage;
         apart = apart && ys[i] != x;
         for (int j = 0; j < i; j++) one = one && ys[i] != ys[j];
     }
-    if (rows == 1 && one && apart && k <= 2048 && kri::pro_fusable(k)) {
+    if (rows == 1 && one && apart && k <= 2048 && k * k * outs < (size_t(3) << 34) && kri::pro_fusable(k)) {
         int rc = ensure_workspace(c, 1, k);
         if (rc) return rc;
         HIPCHK(c, kr::launch_project_pro(c->stream, sem_for_project(*ws[0]), ws, yp, n, 3, xb->p, nullptr, nullptr,

@@ -49,6 +49,34 @@ def test_projections_and_their_workspace(storage, dim, rows):
     hip.close()
 
 
+# a single row over many outputs: 2048 x 12288 in all is the first that is
+# quantized before the launch (as gate and up of 6144), 12256 the last inside it
+@pytest.mark.parametrize("storage", ["q8_0", "q8_0x4"])
+@pytest.mark.parametrize("gate,up", [(6144, 6112), (6144, 6144)])
+def test_one_row_over_many_outputs(storage, gate, up):
+    dim = 2048
+    rng = np.random.default_rng(gate + up)
+    small = rng.normal(0, 0.02, size=(64, dim)).astype(np.float32)
+    # every 64 rows of the oracle's matrix again: its projection repeats too
+    ms = O.Matrix(small, storage)
+    big = {n: O.Matrix(np.resize(small, (w, dim)), storage) for n, w in (("gate", gate), ("up", up))}
+    hip = K.open("hip")
+    h = {n: hip.upload_matrix(product_matrix(m)) for n, m in big.items()}
+    emb = hip.upload_matrix(product_matrix(ms))
+    hip.bind_handles(emb, 0xFFFFFFFF, [h])
+    hip.prepare(None, K.KvSpec(1, 64, 16))
+    x = rng.normal(size=(1, dim)).astype(np.float32)
+    want = ms.project_cpu(x).ravel()
+    y = {"gate": hip.alloc(gate), "up": hip.alloc(up)}
+    hip.project_gate_up(0, hip.upload(x), y["gate"], y["up"], 1)
+    for n, w in (("gate", gate), ("up", up)):
+        assert_bits_equal(hip.read(y[n], w), np.resize(want, w), n)
+    z = hip.alloc(gate)
+    hip.matmul_quantized(h["gate"], z, 1)
+    assert_bits_equal(hip.read(z, gate), np.resize(want, gate), "from the workspace")
+    hip.close()
+
+
 @pytest.mark.parametrize("storage,lens", [("q8_0", [3, 0, 9, 1, 0]), ("q8_0x4", [1, 0, 40]), ("q8_0", [0, 0]),
                                           ("q8_0", [70, 60])])
 def test_hidden_rows_with_empty_sequences(storage, lens):
